@@ -706,9 +706,10 @@ int32_t run_experts(gtmoe_layer *L, int T, int path, hipStream_t s, float *final
     Workspace &w = L->ws;
     const int bm = path == GTMOE_PATH_BF16 ? mfma_tile_m() : kGemvSlice;
     // upper bound of the tiles / slices over all groups; without dispatch
-    // tables, the shared slices plus two workgroups per routed expert
+    // tables, the shared slices, one row per routed expert and one for every
+    // pass of a slice's tokens that an expert could hold beyond its first
     const bool self = path == GTMOE_PATH_FP32 && L->skipped_dispatch;
-    const int max_tiles = self ? L->S * ((T + bm - 1) / bm) + 2 * L->E
+    const int max_tiles = self ? L->S * ((T + bm - 1) / bm) + L->E + T * L->k / bm
                                : L->S * ((T + bm - 1) / bm) + (T * L->k + bm - 1) / bm + L->E;
     auto set_self = [&](GemvArgs &g) {
         g.self_dispatch = 1;

@@ -3,16 +3,27 @@
 // with the multiply-adds on the matrix cores at fp32-level accuracy.
 //
 // Work split: grid (panels of 64 output rows, token slices of all groups);
-// a workgroup's NW waves share one panel and split its K range between them
-// (NW = 4 or 8).
+// a workgroup's NW waves share one panel and split its K range between them,
+// each with RING chunks of weights and tokens in flight.
 // Lane l of a wave owns row l of the panel, so with the panel layout of the
 // weights every 16-byte load of the wave reads 1 KiB of codes contiguously.
 //
 // Arithmetic: v_mfma_f32_4x4x4_16b_bf16 holds 16 independent 4x4x4
-// products; block b of it multiplies 4 tokens (A, broadcast from lanes 0-3)
-// by 4 k-values of rows 4b..4b+3 (B, one row per lane), so a wave computes
-// 4 tokens x 64 rows per instruction and lane l ends up holding row l's dot
-// products for the 4 tokens -- no cross-lane reduction.  Weight codes are
+// products; block b of it multiplies 4 tokens (A) by 4 k-values of rows
+// 4b..4b+3 (B, one row per lane), so a wave computes 4 tokens x 64 rows per
+// instruction and lane l ends up holding row l's dot products for the 4
+// tokens -- no cross-lane reduction.  The instruction can broadcast the A of
+// any one block to all of them (CBSZ, ABID), so one register pair holds a
+// token quad's values for 16 steps, step b in lanes 4b .. 4b + 3: the tokens
+// travel in the weights' register ring, split where they are used, and need
+// no LDS, no staging pass and no barrier before the main loop (they were
+// staged in LDS and read back four times per scale block and quad: with the
+// four-wave workgroups this allows, 2048 -> 1024 FP4 gate/up over 64 tokens
+// and 64 + 1 experts went 46.2 -> 41 us, down 26.6 -> 24.3; over 113 tokens
+// 59.9 -> 51.5 and 31.2 -> 28.6; 1024 -> 2048 Int8, 16 experts, 32 tokens
+// 19.2 -> 18.3 and 13.3 -> 12.2).  What bounds it now is the load path: with
+// the arithmetic left out the same loads take 41.5 us, without the tokens'
+// loads 37.8.  Weight codes are
 // exact in bf16 (Int8 magnitudes <= 127, e2m1 values); the tokens are split
 // as x = hi + lo with hi = bf16(x) and lo = bf16(x - hi), which represents
 // x to about 2^-17 relative, and both halves go through the MFMA with fp32
@@ -41,11 +52,11 @@ template <int PREC>
 struct Chunk;
 template <>
 struct Chunk<kInt8> {
-    static constexpr int U = 2, CB = 2;  // 32 values
+    static constexpr int U = 4, CB = 4;  // 64 values
 };
 template <>
 struct Chunk<kFP4> {
-    static constexpr int U = 1, CB = 2;  // 32 values
+    static constexpr int U = 2, CB = 4;  // 64 values
 };
 template <>
 struct Chunk<kFloat32> {
@@ -57,15 +68,11 @@ struct ChunkRegs {
     uint4 c[MATS][Chunk<PREC>::U];
     float s[MATS][Chunk<PREC>::CB];
 };
-
-// Chunks in flight per wave (register ring): three for FP4 gate/up, whose
-// chunks are half the bytes of Int8's (C5 decode gate/up 1183 -> 1158 us per
-// step), two otherwise (a third chunk measured slower for Int8).
-template <int PREC, int MATS, int NQ>
-constexpr int ring_depth()
-{
-    return PREC == kFP4 && MATS == 2 ? 3 : 2;
-}
+// the lane's four values of its token of every quad
+template <int NQ>
+struct TokenRegs {
+    float4 x[NQ];
+};
 
 // One weight matrix's panel as buffer resources: the panel's codes (64 rows
 // side by side in 16-byte units) and its scales.  The resources live in
@@ -152,29 +159,16 @@ __device__ __forceinline__ void weights_step_f32(const uint4 (&c)[Chunk<kFloat32
     lo = as_s16x4(l01, l23);
 }
 
+// 4 tokens x 64 rows: every block takes its A (4 tokens x 4 k-values) from
+// block ABID, lanes 4 ABID .. 4 ABID + 3 (CBSZ = 4).
+template <int ABID>
 __device__ __forceinline__ f32x4 mfma4(s16x4 a, s16x4 b, f32x4 c)
 {
-    // CBSZ = 4, ABID = 0: block 0's A (lanes 0-3, the tokens) is used by
-    // all 16 blocks
-    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(a, b, c, 4, 0, 0);
+    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(a, b, c, 4, ABID, 0);
 }
 
 // x * sigmoid(x) with the hardware exp and reciprocal (about 1 ulp each)
 __device__ __forceinline__ float silu(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
-
-// The staged tokens: for every group of 8 k-values, NT tokens' bf16 hi
-// values (16 bytes each), then the same for lo.  Lane reads of one token's
-// 16 bytes for tokens 4q..4q+3 are contiguous and shared by the other lanes.
-template <int NT>
-struct Staged {
-    const uint4 *hi;
-    const uint4 *lo;
-    __device__ __forceinline__ void read(int g8, int t, uint4 &h, uint4 &l) const
-    {
-        h = hi[g8 * NT + t];
-        l = lo[g8 * NT + t];
-    }
-};
 
 // Codes (and scales) of chunk ch of the lane's row, for every matrix.  A
 // chunk of CB blocks starts at block ch*CB; its scales are CB consecutive
@@ -210,76 +204,124 @@ __device__ __forceinline__ void load_chunk(ChunkRegs<PREC, MATS> &r, const Panel
     }
 }
 
-// One step of one block: A operands of the NQ token quads for k-values
-// 4S..4S+3, against every matrix.
-template <int PREC, int MATS, int NQ, int J, int S>
-__device__ __forceinline__ void block_step(const ChunkRegs<PREC, MATS> &r, const uint4 (&ah)[NQ],
-                                           const uint4 (&al)[NQ], f32x4 (&blk)[MATS][NQ])
+template <int PREC, int NQ>
+__device__ __forceinline__ void load_tokens(TokenRegs<NQ> &r, __amdgpu_buffer_rsrc_t xin, const uint32_t (&xo)[NQ], int ch)
 {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        const s16x4 xh = (S & 1) ? as_s16x4(ah[q].z, ah[q].w) : as_s16x4(ah[q].x, ah[q].y);
-        const s16x4 xl = (S & 1) ? as_s16x4(al[q].z, al[q].w) : as_s16x4(al[q].x, al[q].y);
+    for (int q = 0; q < NQ; ++q)
+        r.x[q] = __builtin_bit_cast(
+            float4, __builtin_amdgcn_raw_buffer_load_b128(xin, xo[q], ch * (Chunk<PREC>::CB * 64), 0));
+}
+
+// Panel `panel` of group g as buffer resources.
+template <int PREC, bool GATEUP, int MATS>
+__device__ __forceinline__ void panel_src(const GemvArgs &a, int g, int panel, PanelSrc (&src)[MATS])
+{
 #pragma unroll
-        for (int m = 0; m < MATS; ++m) {
-            if constexpr (PREC == kFloat32) {
-                s16x4 wh, wl;
-                weights_step_f32<S>(r.c[m], wh, wl);
-                blk[m][q] = mfma4(xh, wh, blk[m][q]);
-                blk[m][q] = mfma4(xl, wh, blk[m][q]);
-                blk[m][q] = mfma4(xh, wl, blk[m][q]);
-            } else {
-                const s16x4 w = weights_step<PREC, J, S>(r.c[m]);
-                blk[m][q] = mfma4(xh, w, blk[m][q]);
-                blk[m][q] = mfma4(xl, w, blk[m][q]);
-            }
-        }
+    for (int m = 0; m < MATS; ++m) {
+        const int pm = GATEUP ? panel : panel + m;
+        const bool in_matrix = pm * 64 < a.rows;  // the last workgroup's sets may lie past the rows
+        const size_t wpanel = (size_t)pm * 64 * a.row_bytes;
+        const int wbytes = in_matrix ? 64 * a.row_bytes : 0;  // past the rows: every load reads zeros
+        const size_t spanel = (size_t)pm * 64 * a.nblocks;
+        const int sbytes = in_matrix ? 64 * a.nblocks * 4 : 0;
+        src[m].codes = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<char *>(reinterpret_cast<const char *>(GATEUP && m ? a.w1 : a.w0)) + (size_t)g * a.w_group_stride + wpanel,
+            0, wbytes, kRawBufferWord3);
+        if constexpr (PREC != kFloat32)
+            src[m].scales = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float *>(GATEUP && m ? a.s1 : a.s0) + (size_t)g * a.s_group_stride + spanel, 0, sbytes,
+                kRawBufferWord3);
+    }
+}
+
+// Step S (four k-values) of block J of a chunk: the hi and lo halves of every
+// token quad against every matrix.  All hi products come before all lo ones,
+// so that an instruction seldom waits for the one before it.
+template <int PREC, int MATS, int NQ, int J, int S>
+__device__ __forceinline__ void block_step(const ChunkRegs<PREC, MATS> &r, const s16x4 (&xh)[NQ],
+                                           const s16x4 (&xl)[NQ], f32x4 (&blk)[MATS][NQ])
+{
+    constexpr int ABID = 4 * J + S;
+    s16x4 wh[MATS], wl[MATS];
+#pragma unroll
+    for (int m = 0; m < MATS; ++m) {
+        if constexpr (PREC == kFloat32) weights_step_f32<S>(r.c[m], wh[m], wl[m]);
+        else wh[m] = weights_step<PREC, J, S>(r.c[m]);
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int m = 0; m < MATS; ++m) blk[m][q] = mfma4<ABID>(xh[q], wh[m], blk[m][q]);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int m = 0; m < MATS; ++m) blk[m][q] = mfma4<ABID>(xl[q], wh[m], blk[m][q]);
+    if constexpr (PREC == kFloat32) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+            for (int m = 0; m < MATS; ++m) blk[m][q] = mfma4<ABID>(xh[q], wl[m], blk[m][q]);
     }
 }
 
 template <int PREC, int MATS, int NQ, int J>
-__device__ __forceinline__ void chunk_block(const ChunkRegs<PREC, MATS> &r, const Staged<4 * NQ> &xs, int g8,
-                                            int tl, f32x4 (&acc)[MATS][NQ])
+__device__ __forceinline__ void chunk_block(const ChunkRegs<PREC, MATS> &r, const s16x4 (&xh)[NQ],
+                                            const s16x4 (&xl)[NQ], f32x4 (&blk)[MATS][NQ])
 {
-    f32x4 blk[MATS][NQ];
 #pragma unroll
     for (int m = 0; m < MATS; ++m)
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) blk[m][q] = PREC == kFloat32 ? acc[m][q] : f32x4{0.f, 0.f, 0.f, 0.f};
-    uint4 ah[NQ], al[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) xs.read(g8, 4 * q + tl, ah[q], al[q]);
-    block_step<PREC, MATS, NQ, J, 0>(r, ah, al, blk);
-    block_step<PREC, MATS, NQ, J, 1>(r, ah, al, blk);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) xs.read(g8 + 1, 4 * q + tl, ah[q], al[q]);
-    block_step<PREC, MATS, NQ, J, 2>(r, ah, al, blk);
-    block_step<PREC, MATS, NQ, J, 3>(r, ah, al, blk);
+        for (int q = 0; q < NQ; ++q) blk[m][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    block_step<PREC, MATS, NQ, J, 0>(r, xh, xl, blk);
+    block_step<PREC, MATS, NQ, J, 1>(r, xh, xl, blk);
+    block_step<PREC, MATS, NQ, J, 2>(r, xh, xl, blk);
+    block_step<PREC, MATS, NQ, J, 3>(r, xh, xl, blk);
+}
+
+// acc += the block's sums times its scale
+template <int PREC, int MATS, int NQ, int J>
+__device__ __forceinline__ void add_block(const ChunkRegs<PREC, MATS> &r, const f32x4 (&blk)[MATS][NQ],
+                                          f32x4 (&acc)[MATS][NQ])
+{
 #pragma unroll
     for (int m = 0; m < MATS; ++m)
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            if constexpr (PREC == kFloat32) {
-                acc[m][q] = blk[m][q];
-            } else {
-                const float s = r.s[m][J];
+        for (int q = 0; q < NQ; ++q)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[m][q][i] = fmaf(blk[m][q][i], s, acc[m][q][i]);
-            }
-        }
+            for (int i = 0; i < 4; ++i) acc[m][q][i] = fmaf(blk[m][q][i], r.s[m][J], acc[m][q][i]);
 }
 
 template <int PREC, int MATS, int NQ>
-__device__ __forceinline__ void compute_chunk(const ChunkRegs<PREC, MATS> &r, const Staged<4 * NQ> &xs, int ch,
-                                              int tl, f32x4 (&acc)[MATS][NQ])
+__device__ __forceinline__ void compute_chunk(const ChunkRegs<PREC, MATS> &r, const TokenRegs<NQ> &x, int turn_src,
+                                              f32x4 (&acc)[MATS][NQ])
 {
-    constexpr int CB = Chunk<PREC>::CB;
-    const int g8 = ch * CB * 2;  // groups of 8 k-values
-    chunk_block<PREC, MATS, NQ, 0>(r, xs, g8, tl, acc);
-    if constexpr (CB > 1) chunk_block<PREC, MATS, NQ, 1>(r, xs, g8 + 2, tl, acc);
-    if constexpr (CB > 2) {
-        chunk_block<PREC, MATS, NQ, 2>(r, xs, g8 + 4, tl, acc);
-        chunk_block<PREC, MATS, NQ, 3>(r, xs, g8 + 6, tl, acc);
+    s16x4 xh[NQ], xl[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        uint32_t h01, l01, h23, l23;
+        split_pair(x.x[q].x, x.x[q].y, h01, l01);
+        split_pair(x.x[q].z, x.x[q].w, h23, l23);
+        auto turn = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_bpermute(turn_src, (int)v); };
+        xh[q] = as_s16x4(turn(h01), turn(h23));
+        xl[q] = as_s16x4(turn(l01), turn(l23));
+    }
+    if constexpr (PREC == kFloat32) {
+        block_step<PREC, MATS, NQ, 0, 0>(r, xh, xl, acc);
+        block_step<PREC, MATS, NQ, 0, 1>(r, xh, xl, acc);
+        block_step<PREC, MATS, NQ, 0, 2>(r, xh, xl, acc);
+        block_step<PREC, MATS, NQ, 0, 3>(r, xh, xl, acc);
+    } else {
+        // a block's sums are scaled while the next block's products run
+        f32x4 blk[2][MATS][NQ];
+        chunk_block<PREC, MATS, NQ, 0>(r, xh, xl, blk[0]);
+        chunk_block<PREC, MATS, NQ, 1>(r, xh, xl, blk[1]);
+        add_block<PREC, MATS, NQ, 0>(r, blk[0], acc);
+        chunk_block<PREC, MATS, NQ, 2>(r, xh, xl, blk[0]);
+        add_block<PREC, MATS, NQ, 1>(r, blk[1], acc);
+        chunk_block<PREC, MATS, NQ, 3>(r, xh, xl, blk[1]);
+        add_block<PREC, MATS, NQ, 2>(r, blk[0], acc);
+        add_block<PREC, MATS, NQ, 3>(r, blk[1], acc);
     }
 }
 
@@ -312,120 +354,66 @@ __device__ __forceinline__ int slice_out_row(const GemvArgs &a, const SliceSrc &
     else return sl.s * a.T + sl.t0 + t;
 }
 
-// One slice of M <= 4*NQ tokens of group g against panels panel0 ..
-// panel0 + PPW - 1: the NW waves are PPW sets of WPP = NW / PPW, set pi on
-// panel panel0 + pi, its waves splitting K; the sets share the staged tokens.
-template <int PREC, bool GATEUP, int NW, int NQ, int MODE, int PPW>
+// One slice of M <= 4*NQ tokens of group g against one panel of gate and up
+// rows, or against MATS panels of down rows side by side; the workgroup's
+// waves split K.
+template <int PREC, bool GATEUP, int NQ, int MODE, int MATS, int NW, int RING>
 __device__ __forceinline__ void run_slice(const GemvArgs &a, char *lds, int g, const SliceSrc &sl, int M,
-                                          int panel0)
+                                          int panel)
 {
-    static_assert(NW % PPW == 0, "whole sets of waves per panel");
-    constexpr int WPP = NW / PPW;
-    constexpr int NT = 4 * NQ;
-    constexpr int MATS = GATEUP ? 2 : 1;
     constexpr int CB = Chunk<PREC>::CB;
-    // the empty asm hides where tid comes from, so that a caller's loop over
-    // slices cannot hoist the lane-dependent set-up out of the loop and keep
-    // it live across the main loop (that costs about 16 VGPRs)
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
+    const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kp = a.nblocks * 16;
-    const int ng8 = kp / 8;
 
-    // this wave's panel and chunks of K; the first chunks' loads (and the
-    // epilogue's biases) are issued before the token rows are staged
-    const int pi = wave / WPP, kw = wave - pi * WPP;
-    const int panel = panel0 + pi;
-    const bool in_matrix = panel * 64 < a.rows;  // the last workgroup's sets may lie past the rows
+    // this wave's chunks of K
     const int nch = a.nblocks / CB;
-    const int c0 = kw * nch / WPP, c1 = (kw + 1) * nch / WPP;
+    const int c0 = wave * nch / NW, c1 = (wave + 1) * nch / NW;
     PanelSrc src[MATS];
-    {
-        const size_t wpanel = (size_t)panel * 64 * a.row_bytes;
-        const int wbytes = in_matrix ? 64 * a.row_bytes : 0;  // past the rows: every load reads zeros
-        src[0].codes = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<char *>(reinterpret_cast<const char *>(a.w0)) + (size_t)g * a.w_group_stride + wpanel, 0, wbytes,
-            kRawBufferWord3);
-        if constexpr (GATEUP)
-            src[1].codes = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<char *>(reinterpret_cast<const char *>(a.w1)) + (size_t)g * a.w_group_stride + wpanel, 0,
-                wbytes, kRawBufferWord3);
-        if constexpr (PREC != kFloat32) {
-            const size_t spanel = (size_t)panel * 64 * a.nblocks;
-            const int sbytes = in_matrix ? 64 * a.nblocks * 4 : 0;
-            src[0].scales = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float *>(a.s0) + (size_t)g * a.s_group_stride + spanel, 0, sbytes, kRawBufferWord3);
-            if constexpr (GATEUP)
-                src[1].scales = __builtin_amdgcn_make_buffer_rsrc(
-                    const_cast<float *>(a.s1) + (size_t)g * a.s_group_stride + spanel, 0, sbytes, kRawBufferWord3);
-        }
-    }
+    panel_src<PREC, GATEUP, MATS>(a, g, panel, src);
     const uint32_t vo = (uint32_t)lane * 16;
 
-    // The slice's tokens for this wave's K range (groups of 8 k-values
-    // [g0, g0 + gn)) are staged as bf16 hi / lo by the PPW waves that share
-    // the range: one wave (PPW = 1) needs no workgroup barrier before its
-    // main loop.  Item i of a lane is token lane % NT (64 is a multiple of
-    // NT) at group g0 + idx / NT, idx = lane + 64 (pi + PPW i): the lanes'
-    // 16-byte LDS stores are contiguous.  The token loads are issued before
-    // the weight prefetch, the conversion after it, so the wait for the
-    // tokens overlaps the first weight chunks' latency.  Padding tokens
+    // tokens: with NB = 4 CB steps per chunk, lane NB t + b loads the four
+    // k-values of step b of token t of each quad (whole cache lines; lanes
+    // past 4 NB repeat), and once split, lane 4 b + t fetches them from it,
+    // where the matrix instruction of step b broadcasts its A from (loading
+    // them there directly touches four rows per 64 bytes: down 26.4 -> 25.5
+    // us, 33.4 -> 31.3 at 113 tokens, 2048 x 1024 FP4 rows).  Padding tokens
     // (t >= M) read past the input buffer and get zeros.
-    const int g0 = c0 * CB * 2, gn = (c1 - c0) * CB * 2;
-    const int items = NT * gn;
-    const int ipl = (items + 64 * PPW - 1) / (64 * PPW);  // items per lane
-    auto item = [&](int i) { return lane + 64 * (pi + PPW * i); };
-    const int t = lane % NT;
-    uint32_t rowoff = 0x80000000u;  // past the buffer: zeros
-    if (t < M) rowoff = (uint32_t)slice_in_row<GATEUP, MODE>(a, sl, t) * (uint32_t)a.ld_in * 4u;
     const __amdgpu_buffer_rsrc_t xin = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float *>(a.in), 0, (int)(a.in_rows * a.ld_in * 4), kRawBufferWord3);
-    auto token_off = [&](int idx) {
-        return idx < items ? rowoff + (uint32_t)(g0 + idx / NT) * 32u : 0x80000000u;
-    };
-    auto stage = [&](int idx, const float4 &v0, const float4 &v1, uint4 *xhi, uint4 *xlo) {
-        uint4 h, l;
-        split_pair(v0.x, v0.y, h.x, l.x);
-        split_pair(v0.z, v0.w, h.y, l.y);
-        split_pair(v1.x, v1.y, h.z, l.z);
-        split_pair(v1.z, v1.w, h.w, l.w);
-        const int at = (g0 + idx / NT) * NT + t;
-        xhi[at] = h;
-        xlo[at] = l;
-    };
-    // the first kEarly items per lane go ahead of the weight prefetch (all
-    // of them up to 2 KiB of K per wave); any others are staged after it
-    constexpr int kEarly = 2;
-    float4 xv[kEarly][2];
+    uint32_t xo[NQ];
 #pragma unroll
-    for (int i = 0; i < kEarly; ++i) {
-        if (i < ipl) {  // wave-uniform
-            const uint32_t off = token_off(item(i));
-            xv[i][0] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xin, off, 0, 0));
-            xv[i][1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xin, off, 16, 0));
-        }
+    for (int q = 0; q < NQ; ++q) {
+        const int t = 4 * q + ((lane / (4 * CB)) & 3);
+        xo[q] = 0x80000000u;  // past the buffer: zeros
+        if (t < M)
+            xo[q] = (uint32_t)slice_in_row<GATEUP, MODE>(a, sl, t) * (uint32_t)a.ld_in * 4u +
+                    (uint32_t)(lane & (4 * CB - 1)) * 16u;
     }
+    const int turn_src = ((lane & 3) * (4 * CB) + ((lane >> 2) & (4 * CB - 1))) * 4;
 
     // the epilogue's biases are requested before the ring, so that the loads
     // in flight at the main loop's entry are the ring's alone, in ring order,
     // as on its back edge
     const int row = panel * 64 + lane;
-    const bool writer = kw < 4 && row < a.rows;
+    const bool writer = wave < 4 && row < a.rows;
     float bias[MATS];
 #pragma unroll
-    for (int m = 0; m < MATS; ++m) bias[m] = writer ? (m == 0 ? a.b0 : a.b1)[(size_t)g * a.rows + row] : 0.f;
+    for (int m = 0; m < MATS; ++m) {
+        const int rm = GATEUP ? row : min(row + 64 * m, a.rows - 1);
+        bias[m] = writer ? (GATEUP && m ? a.b1 : a.b0)[(size_t)g * a.rows + rm] : 0.f;
+    }
 
-    constexpr int kDepth = ring_depth<PREC, MATS, NQ>();
     // Every load of the ring is issued unconditionally, so that the compiler
     // can count the loads in flight and wait for one chunk at a time (loads
     // under a branch make it wait for all of them).  Past the wave's last
     // chunk the ring re-loads that chunk: cache hits, never used.
     const int clast = c1 > c0 ? c1 - 1 : c0;
-    ChunkRegs<PREC, MATS> r[kDepth];
+    ChunkRegs<PREC, MATS> r[RING];
+    TokenRegs<NQ> x[RING];
 #pragma unroll
-    for (int i = 0; i < kDepth; ++i) {
+    for (int i = 0; i < RING; ++i) {
         // the scheduling barriers keep the ring's loads in ring order here
         // and in the loop: the compiler's wait before each chunk must hold
         // for the loads in flight both at the loop's entry and on its back
@@ -433,36 +421,9 @@ __device__ __forceinline__ void run_slice(const GemvArgs &a, char *lds, int g, c
         // would make it wait for the next chunk's loads as well
         __builtin_amdgcn_sched_barrier(0);
         load_chunk<PREC, MATS>(r[i], src, vo, min(c0 + i, clast));
+        load_tokens<PREC, NQ>(x[i], xin, xo, min(c0 + i, clast));
     }
     __builtin_amdgcn_sched_barrier(0);
-
-    uint4 *xhi = reinterpret_cast<uint4 *>(lds);
-    uint4 *xlo = xhi + (size_t)ng8 * NT;
-#pragma unroll
-    for (int i = 0; i < kEarly; ++i) {
-        const int idx = item(i);
-        if (i < ipl && idx < items) stage(idx, xv[i][0], xv[i][1], xhi, xlo);
-    }
-    for (int i = kEarly; i < ipl; ++i) {
-        const int idx = item(i);
-        const uint32_t off = token_off(idx);
-        const float4 v0 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xin, off, 0, 0));
-        const float4 v1 = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xin, off, 16, 0));
-        if (idx < items) stage(idx, v0, v1, xhi, xlo);
-    }
-    // With one panel the wave reads back only what it wrote; LDS operations
-    // of a wave are performed in order, so a wait for its own stores is
-    // enough.  With several, every wave waits for its own stores and then
-    // for the other waves at a bare barrier (no wait for the weight loads in
-    // flight).  The fences keep the compiler from moving LDS accesses across.
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-    if constexpr (PPW == 1) __builtin_amdgcn_wave_barrier();
-    else __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-    const Staged<NT> xs{xhi, xlo};
-    const int tl = lane & 3;
 
     f32x4 acc[MATS][NQ];
 #pragma unroll
@@ -470,31 +431,31 @@ __device__ __forceinline__ void run_slice(const GemvArgs &a, char *lds, int g, c
 #pragma unroll
         for (int q = 0; q < NQ; ++q) acc[m][q] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // ring of kDepth chunk buffers: once chunk ch is computed, its buffer
-    // takes chunk ch + kDepth.  The loop body computes every buffer with no
+    // ring of RING chunk buffers: once chunk ch is computed, its buffer
+    // takes chunk ch + RING.  The loop body computes every buffer with no
     // branch, so the loads in flight on its back edge are exactly the ring's
     // and the compiler waits, before each chunk, for that chunk's loads only
     // (with a conditional compute in the body it also waited for the next
     // buffer's loads, leaving about one chunk in flight); the last
-    // c1 - ch < kDepth chunks, already in the ring, are computed after it.
+    // c1 - ch < RING chunks, already in the ring, are computed after it.
     int ch = c0;
-    for (; ch + kDepth <= c1; ch += kDepth) {
+    for (; ch + RING <= c1; ch += RING) {
 #pragma unroll
-        for (int j = 0; j < kDepth; ++j) {
-            compute_chunk<PREC, MATS, NQ>(r[j], xs, ch + j, tl, acc);
+        for (int j = 0; j < RING; ++j) {
+            compute_chunk<PREC, MATS, NQ>(r[j], x[j], turn_src, acc);
             __builtin_amdgcn_sched_barrier(0);
-            load_chunk<PREC, MATS>(r[j], src, vo, min(ch + j + kDepth, clast));
+            load_chunk<PREC, MATS>(r[j], src, vo, min(ch + j + RING, clast));
+            load_tokens<PREC, NQ>(x[j], xin, xo, min(ch + j + RING, clast));
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 #pragma unroll
-    for (int j = 0; j + 1 < kDepth; ++j)
-        if (ch + j < c1) compute_chunk<PREC, MATS, NQ>(r[j], xs, ch + j, tl, acc);
+    for (int j = 0; j + 1 < RING; ++j)
+        if (ch + j < c1) compute_chunk<PREC, MATS, NQ>(r[j], x[j], turn_src, acc);
 
-    // sum the partial K ranges of each panel through LDS; wave kw < 4 of the
-    // panel's set then finishes tokens 4q + v of every quad, v = kw, kw +
-    // WPP, ... < 4
-    __syncthreads();  // all reads of the staged tokens are done
+    // sum the partial K ranges through LDS; wave w < 4 then finishes token
+    // 4 q + w of every quad
+    static_assert(NW >= 4, "one wave per token of a quad in the epilogue");
     float *red = reinterpret_cast<float *>(lds);
     auto slot = [&](int wv, int m, int q, int i) { return (((wv * MATS + m) * NQ + q) * 4 + i) * 64 + lane; };
 #pragma unroll
@@ -505,17 +466,16 @@ __device__ __forceinline__ void run_slice(const GemvArgs &a, char *lds, int g, c
             for (int i = 0; i < 4; ++i) red[slot(wave, m, q, i)] = acc[m][q][i];
     __syncthreads();
     if (!writer) return;
-    for (int tq = kw; tq < 4; tq += WPP)
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int t = 4 * q + tq;
+        const int t = 4 * q + wave;
         if (t >= M) continue;
         float v[MATS];
 #pragma unroll
         for (int m = 0; m < MATS; ++m) {
             float s = 0.f;
 #pragma unroll
-            for (int wv = 0; wv < WPP; ++wv) s += red[slot(pi * WPP + wv, m, q, tq)];
+            for (int wv = 0; wv < NW; ++wv) s += red[slot(wv, m, q, wave)];
             v[m] = s;
         }
         const size_t orow = (size_t)slice_out_row<MODE>(a, sl, t) * a.ld_out;
@@ -523,6 +483,9 @@ __device__ __forceinline__ void run_slice(const GemvArgs &a, char *lds, int g, c
         if (a.raw) {  // the bare products (the adapter path adds its terms and the bias)
             *out = v[0];
             if constexpr (GATEUP) a.raw_up[orow + row] = v[MATS - 1];
+            else if constexpr (MATS == 2) {
+                if (row + 64 < a.rows) out[64] = v[1];
+            }
         } else if constexpr (GATEUP) {
             float gv = v[0] + bias[0];
             float uv = v[1] + bias[MATS - 1];
@@ -550,10 +513,15 @@ __device__ __forceinline__ void run_slice(const GemvArgs &a, char *lds, int g, c
                         if (a.chosen[(size_t)tk * a.k + j] == e) wgt = a.gates32[(size_t)tk * a.k + j];
                 }
             }
-            __hip_atomic_fetch_add(a.final_out + (size_t)tk * a.rows + row, wgt * (v[0] + bias[0]), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int m = 0; m < MATS; ++m)
+                if (row + 64 * m < a.rows)
+                    __hip_atomic_fetch_add(a.final_out + (size_t)tk * a.rows + row + 64 * m, wgt * (v[m] + bias[m]),
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-            *out = v[0] + bias[0];
+#pragma unroll
+            for (int m = 0; m < MATS; ++m)
+                if (row + 64 * m < a.rows) out[64 * m] = v[m] + bias[m];
         }
     }
 }
@@ -563,8 +531,8 @@ __device__ __forceinline__ void run_slice(const GemvArgs &a, char *lds, int g, c
 // blockIdx.x = panel of 64 output rows, blockIdx.y = token slice (the
 // dispatch wrote the slice count and a (group, first position, positions)
 // descriptor per slice; slices past the last exit).
-template <int PREC, bool GATEUP, int NW, bool SELF, int PPW>
-__global__ __launch_bounds__(64 * NW) void gemv_kernel(GemvArgs a)
+template <int PREC, bool GATEUP, bool SELF, int MATS, int NW, int RING>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 4) void gemv_kernel(GemvArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int y = blockIdx.y;
@@ -574,9 +542,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(GemvArgs a)
         if (y >= nslices) return;    // workgroup-uniform
         const SliceSrc sl{kByPosition, dsc.y, nullptr, 0, 0};
         if (dsc.z <= 0) return;  // workgroup-uniform
-        const int panel0 = blockIdx.x * PPW;
-        if (dsc.z <= 4) run_slice<PREC, GATEUP, NW, 1, kByPosition, PPW>(a, lds, dsc.x, sl, dsc.z, panel0);
-        else run_slice<PREC, GATEUP, NW, 2, kByPosition, PPW>(a, lds, dsc.x, sl, dsc.z, panel0);
+        const int panel0 = blockIdx.x * (GATEUP ? 1 : MATS);
+        if (dsc.z <= 4) run_slice<PREC, GATEUP, 1, kByPosition, MATS, NW, RING>(a, lds, dsc.x, sl, dsc.z, panel0);
+        else run_slice<PREC, GATEUP, 2, kByPosition, MATS, NW, RING>(a, lds, dsc.x, sl, dsc.z, panel0);
         return;
     } else {
         const int nsh = a.S * a.shared_slices;
@@ -584,24 +552,60 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(GemvArgs a)
             const int s = y / a.shared_slices;
             const SliceSrc sl{kShared, 0, nullptr, (y - s * a.shared_slices) * kGemvSlice, s};
             const int m = min(kGemvSlice, a.T - sl.t0);
-            const int panel0 = blockIdx.x * PPW;
-            if (m <= 4) run_slice<PREC, GATEUP, NW, 1, kShared, PPW>(a, lds, s, sl, m, panel0);
-            else run_slice<PREC, GATEUP, NW, 2, kShared, PPW>(a, lds, s, sl, m, panel0);
+            const int panel0 = blockIdx.x * (GATEUP ? 1 : MATS);
+            if (m <= 4) run_slice<PREC, GATEUP, 1, kShared, MATS, NW, RING>(a, lds, s, sl, m, panel0);
+            else run_slice<PREC, GATEUP, 2, kShared, MATS, NW, RING>(a, lds, s, sl, m, panel0);
             return;
         }
-        // routed expert e: its entries in token order (the order of the
-        // reference's rowsForExpert, mixtureofexperts.go:175-180), found by
-        // wave 0 with ballots over `chosen` (four loads in flight per
-        // round); this workgroup takes passes par, par + 2, ... of 8
-        // entries.  Rows [nsh, nsh + E) are the first halves, [nsh + E,
-        // nsh + 2E) the second, so the second halves (mostly without work at
-        // decode loads) are dispatched after every first half.
-        const int e = (y - nsh) % a.E, par = (y - nsh) / a.E;  // y < nsh + 2E
+        // routed experts: rows [nsh, nsh + E) are each expert's first 8
+        // entries, the T k / 8 rows after them whatever the experts hold beyond
+        // (at most that many passes of 8 in all): extra row j counts every
+        // expert's entries and takes the j-th further pass in expert order, so
+        // a crowded expert's passes run side by side.
         int *list = reinterpret_cast<int *>(lds + a.list_off);
-        int *count = list + a.T * a.k;
+        int *found = list + a.T * a.k;  // entries of the expert, or the extra row's expert and pass
+        const int n = a.T * a.k;
+        int e = y - nsh, first = 0;
+        if (e >= a.E) {
+            int *hist = found + 2;
+            for (int i = threadIdx.x; i < a.E; i += 64 * NW) hist[i] = 0;
+            __syncthreads();
+            for (int i = threadIdx.x; i < n; i += 64 * NW) atomicAdd(&hist[a.chosen[i]], 1);
+            __syncthreads();
+            if (threadIdx.x < 64) {
+                const int j = e - a.E, lane = threadIdx.x;
+                const int per = (a.E + 63) >> 6, e0 = lane * per, e1 = min(a.E, e0 + per);
+                int more = 0;  // further passes of this lane's experts
+                for (int i = e0; i < e1; ++i) more += max(0, (hist[i] - 1) / kGemvSlice);
+                int before = more;
+#pragma unroll
+                for (int off = 1; off < 64; off <<= 1) {
+                    const int v = __shfl_up(before, off);
+                    if (lane >= off) before += v;
+                }
+                before -= more;
+                if (lane == 63) {
+                    found[0] = before + more > j ? 0 : -1;  // -1: no such pass
+                }
+                for (int i = e0; i < e1; ++i) {
+                    const int m = max(0, (hist[i] - 1) / kGemvSlice);
+                    if (j >= before && j < before + m) {
+                        found[1] = i * 64 + (j - before + 1);  // T <= 64: at most 8 passes
+                    }
+                    before += m;
+                }
+            }
+            __syncthreads();
+            if (found[0] < 0) return;  // workgroup-uniform
+            e = __builtin_amdgcn_readfirstlane(found[1] >> 6);
+            first = __builtin_amdgcn_readfirstlane(found[1] & 63) * kGemvSlice;
+            __syncthreads();  // before the list overwrites what was read
+        }
+        // expert e's entries in token order (the order of the reference's
+        // rowsForExpert, mixtureofexperts.go:175-180), found by wave 0 with
+        // ballots over `chosen` (four loads in flight per round)
         if (threadIdx.x < 64) {
             const int lane = threadIdx.x;
-            const int n = a.T * a.k;
             int c = 0;
             for (int b0 = 0; b0 < n; b0 += 256) {
                 int ch[4];
@@ -616,19 +620,16 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(GemvArgs a)
                     c += __popcll(bal);
                 }
             }
-            if (lane == 0) *count = c;
+            if (lane == 0) *found = c;
         }
         __syncthreads();
-        const int c = __builtin_amdgcn_readfirstlane(*count);
-        for (int first = par * kGemvSlice; first < c; first += 2 * kGemvSlice) {
-            const SliceSrc sl{kByEntry, 0, list + first, 0, 0};
-            const int m = min(kGemvSlice, c - first);
-            int g = a.S + e, panel0 = blockIdx.x * PPW;
-            asm volatile("" : "+s"(g), "+s"(panel0));  // as for tid in run_slice
-            if (m <= 4) run_slice<PREC, GATEUP, NW, 1, kByEntry, PPW>(a, lds, g, sl, m, panel0);
-            else run_slice<PREC, GATEUP, NW, 2, kByEntry, PPW>(a, lds, g, sl, m, panel0);
-            __syncthreads();  // the next pass re-stages the LDS
-        }
+        const int c = __builtin_amdgcn_readfirstlane(*found);
+        if (c <= first) return;  // workgroup-uniform
+        const SliceSrc sl{kByEntry, 0, list + first, 0, 0};
+        const int m = min(kGemvSlice, c - first);
+        const int panel0 = blockIdx.x * (GATEUP ? 1 : MATS);
+        if (m <= 4) run_slice<PREC, GATEUP, 1, kByEntry, MATS, NW, RING>(a, lds, a.S + e, sl, m, panel0);
+        else run_slice<PREC, GATEUP, 2, kByEntry, MATS, NW, RING>(a, lds, a.S + e, sl, m, panel0);
     }
 }
 
@@ -841,46 +842,36 @@ __global__ __launch_bounds__(256) void gemv_few_kernel(GemvArgs a)
 
 namespace {
 
-// LDS: the staged tokens (2 x 2 bytes per k-value and token) or the
-// cross-wave partial sums, whichever is larger.
-size_t gemv_lds_bytes(int nblocks, bool gateup, int nw)
+// LDS: the cross-wave partial sums.
+size_t gemv_lds_bytes(int mats, int nw)
 {
-    const size_t staged = (size_t)nblocks * 16 * 2 * 2 * kGemvSlice;
-    const size_t red = (size_t)nw * (gateup ? 2 : 1) * 2 * 4 * 64 * sizeof(float);
-    return staged > red ? staged : red;
+    return (size_t)nw * mats * 2 * 4 * 64 * sizeof(float);
 }
 
-template <int PREC, bool GATEUP, int NW, int PPW = 1>
-hipError_t launch_nw(const GemvArgs &a0, int max_slices, hipStream_t s)
+template <int PREC, bool GATEUP, int MATS, int NW, int RING>
+hipError_t launch_panels(const GemvArgs &a0, int max_slices, hipStream_t s)
 {
     GemvArgs a = a0;
-    size_t lds = gemv_lds_bytes(a.nblocks, GATEUP, NW);
+    size_t lds = gemv_lds_bytes(MATS, NW);
     if (a.self_dispatch) {
-        // the routed expert's entry list and its length after the slice's LDS
+        // after the slice's LDS: the routed expert's entry list, its length (two
+        // ints) and an extra row's count per expert
         a.list_off = (int)((lds + 15) / 16 * 16);
-        lds = (size_t)a.list_off + ((size_t)a.T * a.k + 1) * sizeof(int);
+        lds = (size_t)a.list_off + ((size_t)a.T * a.k + 2 + a.E) * sizeof(int);
     }
     if (lds > 160 * 1024) return hipErrorInvalidValue;
-    const void *fn = a.self_dispatch ? reinterpret_cast<const void *>(&gemv_kernel<PREC, GATEUP, NW, true, PPW>)
-                                     : reinterpret_cast<const void *>(&gemv_kernel<PREC, GATEUP, NW, false, PPW>);
+    const void *fn = a.self_dispatch ? reinterpret_cast<const void *>(&gemv_kernel<PREC, GATEUP, true, MATS, NW, RING>)
+                                     : reinterpret_cast<const void *>(&gemv_kernel<PREC, GATEUP, false, MATS, NW, RING>);
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    const dim3 grid((a.rows + 64 * PPW - 1) / (64 * PPW), max_slices);
+    constexpr int kRows = kPanelRows * (GATEUP ? 1 : MATS);  // rows of a workgroup
+    const dim3 grid((a.rows + kRows - 1) / kRows, max_slices);
     if (a.self_dispatch)
-        hipLaunchKernelGGL((gemv_kernel<PREC, GATEUP, NW, true, PPW>), grid, dim3(64 * NW), lds, s, a);
-    else hipLaunchKernelGGL((gemv_kernel<PREC, GATEUP, NW, false, PPW>), grid, dim3(64 * NW), lds, s, a);
+        hipLaunchKernelGGL((gemv_kernel<PREC, GATEUP, true, MATS, NW, RING>), grid, dim3(64 * NW), lds, s, a);
+    else hipLaunchKernelGGL((gemv_kernel<PREC, GATEUP, false, MATS, NW, RING>), grid, dim3(64 * NW), lds, s, a);
     return hipGetLastError();
-}
-
-// Waves per workgroup: eight when K holds at least two chunks per wave,
-// else four (the epilogue's waves).
-template <int PREC>
-int waves_for(const GemvArgs &a)
-{
-    const int nch = a.nblocks / Chunk<PREC>::CB;
-    return nch >= 16 ? 8 : 4;
 }
 
 template <bool GATEUP, int PREC>
@@ -888,23 +879,31 @@ hipError_t launch_prec(const GemvArgs &a, int max_slices, hipStream_t s)
 {
     static_assert(kGemvSlice <= 8, "at most two token quads per slice");
     if (a.nblocks % Chunk<PREC>::CB) return hipErrorInvalidValue;
-    // a self-dispatching gate/up launch whose experts nearly all have tokens,
-    // over K <= 32 chunks: four waves per workgroup (eight chunks each) fit
-    // every busy workgroup at once; eight would leave some for a second round
-    if (GATEUP && a.self_dispatch && a.nblocks / Chunk<PREC>::CB <= 32 && a.T * a.k >= a.E)
-        return launch_nw<PREC, GATEUP, 4>(a, max_slices, s);
-    // Down over many workgroups: two panels per workgroup, which stages its
-    // tokens once for both (the staging was a fifth of the C5 decode down
-    // kernel: 30.0 -> 27.6 us per layer).  With fewer busy workgroups than
-    // two rounds' worth at the halved count the grid would no longer fill
-    // the GPU (a C2-sized layer: 14.5 -> 17.9 us), so those keep one panel.
-    if (!GATEUP && waves_for<PREC>(a) == 8 && a.rows >= 128) {
-        const long long busy = a.self_dispatch ? (long long)a.S * a.shared_slices + std::min(a.E, a.T * a.k)
-                                               : (long long)max_slices;
-        if ((long long)(a.rows / 128) * busy >= 1024) return launch_nw<PREC, GATEUP, 8, 2>(a, max_slices, s);
+    const long long busy = a.self_dispatch ? (long long)a.S * a.shared_slices + std::min(a.E, a.T * a.k)
+                                           : (long long)max_slices;
+    // Down over many workgroups: a wave takes two panels side by side, so that
+    // its tokens are read and split once for both (2048 x 1024 FP4 rows, 64
+    // experts: 25.6 -> 24.3 us at 64 tokens, 31.1 -> 28.6 us at 113).  With
+    // fewer than two rounds of busy workgroups at the halved count the grid no
+    // longer fills the GPU (1024 x 2048 Int8 rows, 16 experts: 12.2 -> 15.3
+    // us), so those keep one panel per wave.
+    if (!GATEUP && a.rows >= 128 && (long long)(a.rows / 128) * busy >= 1024)
+        return launch_panels<PREC, GATEUP, 2, 4, 2>(a, max_slices, s);
+    constexpr int MATS = GATEUP ? 2 : 1;
+    // Four waves over a ring of two chunks, except where K holds a chunk for
+    // each of eight and these do better: gate/up over fewer than 512 busy
+    // workgroups (Int8 and FP4: eight waves over a ring of one; d = 2048, h =
+    // 1024, 64 + 1 experts over 7 tokens, the layer 48.4 -> 44.9 us in FP4 and
+    // 62.5 -> 58.9 in Int8; over 16 tokens, with twice the workgroups, 54.8
+    // against 59.3 in FP4), and Float32 with K >= 1024 in a self-dispatching
+    // launch (a ring of two; d = 1024, h = 2048, 16 experts over 32 tokens 88.4
+    // -> 82.7; elsewhere it loses: K = 256, 700 tokens 43.7 against 48.6).
+    if constexpr (PREC == kFloat32) {
+        if (a.self_dispatch && a.nblocks >= 64) return launch_panels<PREC, GATEUP, MATS, 8, 2>(a, max_slices, s);
+    } else if (GATEUP && a.nblocks >= 32 && (long long)((a.rows + kPanelRows - 1) / kPanelRows) * busy < 512) {
+        return launch_panels<PREC, GATEUP, MATS, 8, 1>(a, max_slices, s);
     }
-    if (waves_for<PREC>(a) == 8) return launch_nw<PREC, GATEUP, 8>(a, max_slices, s);
-    return launch_nw<PREC, GATEUP, 4>(a, max_slices, s);
+    return launch_panels<PREC, GATEUP, MATS, 4, 2>(a, max_slices, s);
 }
 
 // Up to this many tokens the few-token kernel runs: it streams an expert's
@@ -934,7 +933,7 @@ bool launch_few_tokens(const GemvArgs &a, int precision, hipStream_t s, hipError
 {
     if (!a.self_dispatch || a.T < 1 || a.T > kFewTokens || a.raw || (precision != kInt8 && precision != kFP4))
         return false;
-    if (a.nblocks / Chunk<kInt8>::CB < 16 || a.nblocks * 16 > 4096) return false;
+    if (a.nblocks < 32 || a.nblocks * 16 > 4096) return false;
     const int nunits = a.row_bytes / 16;
     const int R = (long long)(a.rows / 16) * (a.S + a.k) * a.T >= 256 ? 16 : 8;
     if (a.row_bytes % 16 != 0 || nunits % (4 * (64 / R)) != 0) return false;

@@ -582,3 +582,28 @@ def test_stack_routing_outputs_need_one_k(ctx):
         for m in ms:
             m.destroy()
     assert np.all(np.isfinite(x))
+
+
+@pytest.mark.parametrize("prec", [FLOAT32, INT8, FP4])
+@pytest.mark.parametrize("E,k,T", [(1, 1, 9), (4, 2, 8), (4, 2, 17), (64, 4, 64), (200, 3, 33)])
+def test_crowded_experts_in_few_tokens(ctx, prec, E, k, T):
+    """Hash routing with one id on every row but a few: k experts hold nearly
+    every token, so the decode kernels' passes of 8 tokens beyond an expert's
+    first run in the extra workgroups.  K of 9 and 5 chunks of 64 values split
+    unevenly over four and eight waves."""
+    say(f"crowded experts E={E} k={k} T={T} precision {prec}")
+    spec = make_moe(gt.encode_rows, d=576, h=300, E=E, k=k, S=1, precision=prec, seed=31, std=0.05, bias_std=0.02,
+                    use_hash=True)
+    rng = np.random.default_rng(T)
+    x = rng.normal(size=(T, 576))
+    ids = np.full(T, 7, np.int64)
+    ids[::5] = rng.integers(0, 1000, size=len(ids[::5]))
+    m = gt.MixtureOfExperts.from_spec(ctx, spec)
+    try:
+        y = m.forward(x, ids, path=gt.PATH_FP32)
+        r = m.last_routing()
+    finally:
+        m.destroy()
+    ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates)
+    e = rel_err(y, ref.outputs)
+    assert e <= FP32_TOL, e  # the fp32 path's bar: 2^-17 per split token, over fp32 sums
