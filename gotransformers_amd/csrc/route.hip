@@ -969,157 +969,139 @@ hipError_t launch_hash_route(const int64_t *ids, int T, int E, int k, int32_t *c
 // ---------------------------------------------------------------------------
 // Dispatch (mixtureofexperts.go:175-190): per-expert load, exclusive offsets,
 // and a stable permutation -- experts ascending, tokens ascending inside an
-// expert.  The rank of a token inside its expert comes from wave ballots and
-// prefix sums, never from an atomic, so the order is the reference's.  Also
-// fills the position tables the expert kernels use (goff, tok) and the
-// per-group MFMA tile prefix (tile_off).
+// expert.  A token-wave is 64 consecutive tokens; each of its tokens sets its
+// bit in the 64-bit mask of every expert it chose (LDS atomic or: the mask
+// does not depend on the order), so a token's rank among the token-wave's
+// tokens of that expert is the number of bits below its own and the mask's
+// popcount is the count.  No atomic decides an order.  (Ballots of "has this
+// expert" over every (token-wave, expert) pair, twice, took most of the
+// kernels' time: one workgroup, 64 experts, k = 4, 333 tokens 16.3 -> 5.8 us;
+// placement of 4096 tokens, k = 6, 9.5 -> 5.4 us, of 16384 over 128 experts,
+// k = 8, 17.4 -> 10.5.  Three barriers and their round trips are left.)  Also
+// fills the position tables the expert kernels use (goff, tok) and the tiles or
+// slices of every group (tile_off, tile_desc).
 // ---------------------------------------------------------------------------
-constexpr int kScanMax = 1024;  // experts + shared experts handled by the scans
-
-// Exclusive scan of vals[0..n) (n <= 1024) by a 1024-thread workgroup into
-// out[0..n); returns the total.  vals and out may alias.
-__device__ int block_exclusive_scan(const int *vals, int *out, int n, int *wave_sums, int *total_slot)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int v = tid < n ? vals[tid] : 0;
-    int x = v;
-    for (int off = 1; off < 64; off <<= 1) {
-        const int y = __shfl_up(x, off);
-        if (lane >= off) x += y;
-    }
-    if (lane == 63) wave_sums[wave] = x;
-    __syncthreads();
-    if (wave == 0) {
-        int w = lane < 16 ? wave_sums[lane] : 0;
-        int inc = w;
-        for (int off = 1; off < 16; off <<= 1) {
-            const int y = __shfl_up(inc, off);
-            if (lane >= off) inc += y;
-        }
-        if (lane < 16) wave_sums[lane] = inc - w;
-        if (lane == 15) *total_slot = inc;
-    }
-    __syncthreads();
-    if (tid < n) out[tid] = x - v + wave_sums[wave];
-    __syncthreads();
-    return *total_slot;
-}
-
 struct DispatchShared {
-    int cnt[kScanMax];
-    int base[kScanMax];
-    int tiles[kScanMax];
-    int wave_cnt[16][kMaxExperts];
-    int wave_sums[16];
-    int total;
+    int cnt[kMaxExperts];   // entries of an expert
+    int base[kMaxExperts];  // entries of the experts before it
+    int tile[kMaxExperts];  // tiles of the experts before it
+    int tiles;              // tiles of all routed experts
 };
 
-// Group tables from per-expert counts (in sh.cnt) and their exclusive
-// offsets (in sh.base): load, offsets, goff, tile_off and the shared-expert
-// part of tok.
-__device__ void write_group_tables(int T, int k, int E, int S, int bm, DispatchShared &sh, int32_t *__restrict__ load,
-                                   int32_t *__restrict__ offsets, int32_t *__restrict__ goff,
-                                   int32_t *__restrict__ tok, int32_t *__restrict__ tile_off,
+// base and tile from cnt, by one wave (four experts per lane).
+__device__ __forceinline__ void scan_experts(DispatchShared &sh, int E, int bm, int lane)
+{
+    int c[4], n[4], csum = 0, nsum = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = 4 * lane + i;
+        c[i] = e < E ? sh.cnt[e] : 0;
+        n[i] = (c[i] + bm - 1) / bm;
+        csum += c[i];
+        nsum += n[i];
+    }
+    int cx = csum, nx = nsum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int cy = __shfl_up(cx, off), ny = __shfl_up(nx, off);
+        if (lane >= off) {
+            cx += cy;
+            nx += ny;
+        }
+    }
+    if (lane == 63) sh.tiles = nx;
+    cx -= csum;
+    nx -= nsum;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = 4 * lane + i;
+        if (e < E) {
+            sh.base[e] = cx;
+            sh.tile[e] = nx;
+        }
+        cx += c[i];
+        nx += n[i];
+    }
+}
+
+// Group tables from sh (scan_experts done): load, offsets, goff, tile_off and
+// tile_desc.
+__device__ void write_group_tables(int T, int k, int E, int S, int bm, const DispatchShared &sh,
+                                   int32_t *__restrict__ load, int32_t *__restrict__ offsets,
+                                   int32_t *__restrict__ goff, int32_t *__restrict__ tile_off,
                                    int4 *__restrict__ tile_desc)
 {
     const int tid = threadIdx.x;
-    const int G = S + E;
+    const int tps = (T + bm - 1) / bm;  // tiles of a shared expert
     for (int e = tid; e < E; e += blockDim.x) {
-        load[e] = sh.cnt[e];
+        const int m = sh.cnt[e], p = S * T + sh.base[e], t0 = S * tps + sh.tile[e];
+        load[e] = m;
         offsets[e] = sh.base[e];
+        goff[S + e] = p;
+        tile_off[S + e] = t0;
+        // tile -> (group, first position, positions)
+        for (int first = 0, i = t0; first < m; first += bm, ++i)
+            tile_desc[i] = make_int4(S + e, p + first, min(bm, m - first), 0);
     }
-    if (tid == 0) offsets[E] = T * k;
-    for (int g = tid; g < G; g += blockDim.x) {
-        const int m = g < S ? T : sh.cnt[g - S];
-        sh.tiles[g] = (m + bm - 1) / bm;
-        goff[g] = g < S ? g * T : S * T + sh.base[g - S];
-    }
-    if (tid == 0) goff[G] = S * T + T * k;
-    __syncthreads();
-    const int total_tiles = block_exclusive_scan(sh.tiles, sh.tiles, G, sh.wave_sums, &sh.total);
-    for (int g = tid; g < G; g += blockDim.x) {
-        tile_off[g] = sh.tiles[g];
-        const int end = g + 1 < G ? sh.tiles[g + 1] : total_tiles;
-        const int m = g < S ? T : sh.cnt[g - S];
-        const int p = g < S ? g * T : S * T + sh.base[g - S];
-        for (int t = sh.tiles[g]; t < end; ++t) {
-            // tile -> (group, first position, positions)
-            const int first = (t - sh.tiles[g]) * bm;
-            tile_desc[t] = make_int4(g, p + first, min(bm, m - first), 0);
+    for (int i = tid; i < S * tps; i += blockDim.x) {
+        const int g = i / tps, first = (i - g * tps) * bm;
+        if (first == 0) {
+            goff[g] = g * T;
+            tile_off[g] = i;
         }
+        tile_desc[i] = make_int4(g, g * T + first, min(bm, T - first), 0);
     }
-    if (tid == 0) tile_off[G] = total_tiles;
-    for (long long p = tid; p < (long long)S * T; p += blockDim.x) tok[p] = (int32_t)(p % T);
+    if (tid == 0) {
+        offsets[E] = T * k;
+        goff[S + E] = S * T + T * k;
+        tile_off[S + E] = S * tps + sh.tiles;
+    }
 }
 
-// Whole dispatch by one 1024-thread workgroup for T <= 1024; `chosen` may be
-// in LDS.  Tokens form token-waves of 64 (lane = token); the (token-wave,
-// expert) pairs are spread over the 16 waves.  For each pair a ballot of
-// "has this expert" gives the pair's count (pass 1) and every token's rank
-// (pass 2); a per-expert prefix over token-waves in between turns counts into
-// starting positions.  No atomics, and every wave has a share of the work.
-__device__ void dispatch_block(const int32_t *chosen, int T, int k, int E, int S, int bm, int32_t *__restrict__ load,
-                               int32_t *__restrict__ offsets, int32_t *__restrict__ rows, int32_t *__restrict__ pos,
-                               int32_t *__restrict__ goff, int32_t *__restrict__ tok,
-                               int32_t *__restrict__ tile_off, int4 *__restrict__ tile_desc, DispatchShared &sh)
+// Whole dispatch by one 1024-thread workgroup for T <= 1024 (thread = token).
+__device__ void dispatch_block(const int32_t *__restrict__ chosen, int T, int k, int E, int S, int bm,
+                               int32_t *__restrict__ load, int32_t *__restrict__ offsets, int32_t *__restrict__ rows,
+                               int32_t *__restrict__ pos, int32_t *__restrict__ goff, int32_t *__restrict__ tok,
+                               int32_t *__restrict__ tile_off, int4 *__restrict__ tile_desc)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ DispatchShared sh;
+    __shared__ unsigned long long mask[16][kMaxExperts];
+    __shared__ int first[16][kMaxExperts];  // entries of an expert in the token-waves before
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int tw = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ntw = (T + 63) / 64;  // token-waves, <= 16
-    int ntwp = 1;
-    while (ntwp < ntw) ntwp <<= 1;
-    const int wpt = 16 / ntwp;  // waves per token-wave
-    const int tw = wave / wpt, sub = wave % wpt;
-    const int t = tw * 64 + lane;
-    const bool active = tw < ntw;
     int ce[kMaxK];
 #pragma unroll
-    for (int i = 0; i < kMaxK; ++i) ce[i] = (active && t < T && i < k) ? chosen[(size_t)t * k + i] : -1;
-
-    // pass 1: counts per (token-wave, expert)
-    if (active) {
-        for (int e = sub; e < E; e += wpt) {
-            bool has = false;
-#pragma unroll
-            for (int i = 0; i < kMaxK; ++i) has |= ce[i] == e;
-            const unsigned long long b = __ballot(has);
-            if (lane == 0) sh.wave_cnt[tw][e] = __popcll(b);
-        }
-    }
+    for (int i = 0; i < kMaxK; ++i) ce[i] = tid < T && i < k ? chosen[(size_t)tid * k + i] : -1;
+    for (int i = tid; i < ntw * kMaxExperts; i += 1024) mask[i / kMaxExperts][i % kMaxExperts] = 0;
     __syncthreads();
-    // per-expert totals and the prefix over token-waves
-    for (int e = tid; e < E; e += 1024) {
+#pragma unroll
+    for (int i = 0; i < kMaxK; ++i)
+        if (ce[i] >= 0) atomicOr(&mask[tw][ce[i]], 1ull << lane);
+    __syncthreads();
+    if (tid < E) {
         int acc = 0;
-        for (int w = 0; w < ntw; ++w) acc += sh.wave_cnt[w][e];
-        sh.cnt[e] = acc;
-    }
-    __syncthreads();
-    block_exclusive_scan(sh.cnt, sh.base, E, sh.wave_sums, &sh.total);
-    write_group_tables(T, k, E, S, bm, sh, load, offsets, goff, tok, tile_off, tile_desc);
-    for (int e = tid; e < E; e += 1024) {
-        int acc = sh.base[e];
         for (int w = 0; w < ntw; ++w) {
-            const int c = sh.wave_cnt[w][e];
-            sh.wave_cnt[w][e] = acc;
-            acc += c;
+            first[w][tid] = acc;
+            acc += __popcll(mask[w][tid]);
         }
+        sh.cnt[tid] = acc;
     }
     __syncthreads();
-    // pass 2: positions
-    if (active) {
-        for (int e = sub; e < E; e += wpt) {
-            int match = -1;
+    if (tw == 0) scan_experts(sh, E, bm, lane);
+    __syncthreads();
 #pragma unroll
-            for (int i = 0; i < kMaxK; ++i)
-                if (ce[i] == e) match = i;
-            const unsigned long long b = __ballot(match >= 0);
-            if (match >= 0) {
-                const int p = sh.wave_cnt[tw][e] + __popcll(b & ((1ULL << lane) - 1ULL));
-                rows[p] = t;
-                pos[(size_t)t * k + match] = p;
-                tok[(size_t)S * T + p] = t;
-            }
-        }
+    for (int i = 0; i < kMaxK; ++i) {
+        if (ce[i] < 0) continue;
+        const int e = ce[i];
+        const int p = sh.base[e] + first[tw][e] + __popcll(mask[tw][e] & ((1ull << lane) - 1ull));
+        rows[p] = tid;
+        pos[(size_t)tid * k + i] = p;
+        tok[(size_t)S * T + p] = tid;
     }
+    if (tid < T)
+        for (int s = 0; s < S; ++s) tok[(size_t)s * T + tid] = tid;
+    write_group_tables(T, k, E, S, bm, sh, load, offsets, goff, tile_off, tile_desc);
 }
 
 // With pack.n > 0 the same workgroup then gathers pack's parts into
@@ -1132,8 +1114,7 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
                                                         int32_t *__restrict__ tile_off, int4 *__restrict__ tile_desc,
                                                         PackParts pack, uint32_t *__restrict__ pack_dst)
 {
-    __shared__ DispatchShared sh;
-    dispatch_block(chosen, T, k, E, S, bm, load, offsets, rows, pos, goff, tok, tile_off, tile_desc, sh);
+    dispatch_block(chosen, T, k, E, S, bm, load, offsets, rows, pos, goff, tok, tile_off, tile_desc);
     if (pack.n <= 0) return;
     __syncthreads();  // the tables this workgroup wrote are visible to all of it
     uint32_t *out = pack_dst;
@@ -1146,13 +1127,10 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
 }
 
 // Many tokens: chunks of kChunk tokens per workgroup.
-//   count:   per-chunk, per-expert counts            -> chunk_cnt[c][e]
-//   scan:    one workgroup: per-expert totals, offsets, the group tables, and
-//            every chunk's starting position per expert -> chunk_cnt[c][e]
-//   scatter: per chunk, wave ranks + the chunk's base  -> rows, pos, tok
-// kChunk = 128 tokens per chunk: twice the workgroups of 256 for a shorter
-// per-workgroup chain (C3 dispatch 16.5 → 15.6 µs); every placement
-// workgroup reads all chunks' counts, so the chunks are not made smaller.
+//   count:  per-chunk, per-expert counts                -> chunk_cnt[c][e]
+//   place:  per chunk, totals, ranks and the chunk's base -> rows, pos, tok
+// kChunk = 128 tokens per chunk; every placement workgroup reads all chunks'
+// counts, so the chunks are not made smaller.
 // The counts come from the top-k when it runs just before (launch_topk with
 // chunk_cnt), else from dispatch_count_kernel.
 
@@ -1169,13 +1147,12 @@ __global__ __launch_bounds__(kChunk) void dispatch_count_kernel(const int32_t *_
     for (int e = threadIdx.x; e < E; e += kChunk) chunk_cnt[(size_t)blockIdx.x * E + e] = cnt[e];
 }
 
-// Placement of one chunk of kChunk tokens, 16 waves.  Every workgroup sums
-// the per-chunk counts itself (threads split the chunks of each expert), so
-// the totals, the experts' offsets and its own chunk's start need no
-// separate scan launch; workgroup 0 also writes the group tables.  Ranks
-// inside the chunk come from wave ballots, with the (token-wave, expert)
-// pairs spread over the 16 waves.  No atomic decides a position: the LDS
-// atomics only add up counts.
+// Placement of one chunk of kChunk tokens.  Every workgroup sums the
+// per-chunk counts itself (threads split the chunks of each expert), so the
+// totals, the experts' offsets and its own chunk's start need no separate
+// scan launch; workgroup 0 also writes the group tables.  A thread places one
+// (token, slot) entry.  No atomic decides a position: the LDS atomics only
+// add up counts and set the tokens' bits.
 __global__ __launch_bounds__(1024) void dispatch_place_kernel(const int32_t *__restrict__ chosen, int T, int k, int E,
                                                               int S, int bm, int chunks,
                                                               const int32_t *__restrict__ chunk_cnt,
@@ -1185,16 +1162,25 @@ __global__ __launch_bounds__(1024) void dispatch_place_kernel(const int32_t *__r
                                                               int32_t *__restrict__ tile_off,
                                                               int4 *__restrict__ tile_desc)
 {
+    constexpr int kTW = kChunk / 64;  // token-waves of a chunk
+    static_assert(kChunk * kMaxK <= 1024, "an entry per thread");
     __shared__ DispatchShared sh;
     __shared__ int before[kMaxExperts];
-    __shared__ int rank_lds[kChunk][kMaxK];
+    __shared__ unsigned long long mask[kTW][kMaxExperts];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = blockIdx.x;
+    // this thread's entry: token tl of the chunk, slot i
+    const int tl = tid / k, i = tid - tl * k, t = c * kChunk + tl;
+    const bool mine = tl < kChunk && t < T;
+    const int e_mine = mine ? chosen[(size_t)t * k + i] : 0;
     for (int e = tid; e < E; e += 1024) {
         sh.cnt[e] = 0;
         before[e] = 0;
+#pragma unroll
+        for (int w = 0; w < kTW; ++w) mask[w][e] = 0;
     }
     __syncthreads();
+    if (mine) atomicOr(&mask[tl >> 6][e_mine], 1ull << (tl & 63));
     // totals over all chunks and over the chunks before this one
     const int per = 1024 / E;  // threads per expert (E <= 256)
     if (tid < per * E) {
@@ -1216,52 +1202,20 @@ __global__ __launch_bounds__(1024) void dispatch_place_kernel(const int32_t *__r
         atomicAdd(&before[e], bef);
     }
     __syncthreads();
-    block_exclusive_scan(sh.cnt, sh.base, E, sh.wave_sums, &sh.total);
-    if (c == 0) write_group_tables(T, k, E, S, bm, sh, load, offsets, goff, tok, tile_off, tile_desc);
-
-    // ranks inside the chunk: the 16 waves cover the chunk's kChunk / 64
-    // token-waves, kSubsets waves per token-wave; wave w covers token-wave
-    // w / kSubsets and the experts e = w % kSubsets (mod kSubsets)
-    constexpr int kSubsets = 16 / (kChunk / 64);
-    const int tw = wave / kSubsets, sub = wave % kSubsets;
-    const int tl = tw * 64 + lane;
-    const int t = c * kChunk + tl;
-    int ce[kMaxK];
-#pragma unroll
-    for (int i = 0; i < kMaxK; ++i) ce[i] = (t < T && i < k) ? chosen[(size_t)t * k + i] : -1;
-    for (int e = sub; e < E; e += kSubsets) {
-        int match = -1;
-#pragma unroll
-        for (int i = 0; i < kMaxK; ++i)
-            if (ce[i] == e) match = i;
-        const unsigned long long b = __ballot(match >= 0);
-        if (lane == 0) sh.wave_cnt[tw][e] = __popcll(b);
-        if (match >= 0) rank_lds[tl][match] = __popcll(b & ((1ULL << lane) - 1ULL));
-    }
+    if (wave == 0) scan_experts(sh, E, bm, lane);
     __syncthreads();
-    // first position of each (token-wave, expert)
-    for (int e = tid; e < E; e += 1024) {
-        int acc = sh.base[e] + before[e];
+    if (mine) {
+        int p = sh.base[e_mine] + before[e_mine] + __popcll(mask[tl >> 6][e_mine] & ((1ull << (tl & 63)) - 1ull));
 #pragma unroll
-        for (int w = 0; w < kChunk / 64; ++w) {
-            const int n = sh.wave_cnt[w][e];
-            sh.wave_cnt[w][e] = acc;
-            acc += n;
-        }
+        for (int w = 0; w < kTW - 1; ++w)
+            if (w < (tl >> 6)) p += __popcll(mask[w][e_mine]);
+        rows[p] = t;
+        pos[(size_t)t * k + i] = p;
+        tok[(size_t)S * T + p] = t;
     }
-    __syncthreads();
-    if (tid < kChunk) {
-        const int tt = c * kChunk + tid;
-        if (tt < T) {
-            for (int i = 0; i < k; ++i) {
-                const int e = chosen[(size_t)tt * k + i];
-                const int p = sh.wave_cnt[tid >> 6][e] + rank_lds[tid][i];
-                rows[p] = tt;
-                pos[(size_t)tt * k + i] = p;
-                tok[(size_t)S * T + p] = tt;
-            }
-        }
-    }
+    if (tid < kChunk && c * kChunk + tid < T)
+        for (int s = 0; s < S; ++s) tok[(size_t)s * T + c * kChunk + tid] = c * kChunk + tid;
+    if (c == 0) write_group_tables(T, k, E, S, bm, sh, load, offsets, goff, tile_off, tile_desc);
 }
 
 hipError_t launch_dispatch_packed(const int32_t *chosen, int T, int k, int E, int S, int bm, int32_t *load,

@@ -607,3 +607,31 @@ def test_crowded_experts_in_few_tokens(ctx, prec, E, k, T):
     ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates)
     e = rel_err(y, ref.outputs)
     assert e <= FP32_TOL, e  # the fp32 path's bar: 2^-17 per split token, over fp32 sums
+
+
+@pytest.mark.parametrize("T", [1, 63, 65, 128, 1023, 1024, 1025, 1153])
+@pytest.mark.parametrize("E,k", [(1, 1), (7, 5), (65, 3), (256, 8)])
+def test_dispatch_at_the_edges_of_token_waves_and_chunks(ctx, E, k, T):
+    """The dispatch of 64-token waves in one workgroup (up to 1024 tokens) and
+    in chunks of 128 beyond: load, offsets and the stable order, to the bit,
+    and every position's row through a forward with shared experts."""
+    say(f"dispatch edges E={E} k={k} T={T}")
+    rng = np.random.default_rng(1000 * E + T)
+    logits = rng.normal(size=(T, E))
+    logits[:, E // 2] += 3.0  # one expert most tokens choose
+    spec = make_moe(gt.encode_rows, d=8, h=16, E=E, k=k, S=2, precision=INT8, seed=4, std=0.3)
+    x = rng.normal(size=(T, 8))
+    m = gt.MixtureOfExperts.from_spec(ctx, spec)
+    try:
+        got = m.route_from_logits(logits)
+        y = m.forward(x, path=gt.PATH_BF16)
+        r = m.last_routing()
+    finally:
+        m.destroy()
+    for g in (got, r):
+        d = oracle.dispatch(g.chosen, E)
+        assert np.array_equal(g.load, d.load)
+        assert np.array_equal(g.offsets, d.offsets)
+        assert np.array_equal(g.rows, d.rows)
+    ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates)
+    assert rel_err(y, ref.outputs) <= 2e-2  # the bf16 path's bar
