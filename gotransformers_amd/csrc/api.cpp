@@ -575,7 +575,7 @@ int32_t prepare_and_route(gtmoe_layer *L, int T, const Inputs &in, const int64_t
     }
     // the dispatch's per-group tile prefix counts MFMA m-tiles on the bf16
     // path and token slices on the fp32 path
-    const int bm = path == GTMOE_PATH_BF16 ? mfma_tile_m() : kGemvSlice;
+    const int bm = path == GTMOE_PATH_BF16 ? mfma_tile_m(T, L->k, L->E) : kGemvSlice;
     if (fused_route_fits(T, L->k, L->dp)) {
         FusedArgs f{};
         f.x = in.x;
@@ -704,7 +704,7 @@ int32_t run_experts(gtmoe_layer *L, int T, int path, hipStream_t s, float *final
 {
     gtmoe_context *ctx = L->ctx;
     Workspace &w = L->ws;
-    const int bm = path == GTMOE_PATH_BF16 ? mfma_tile_m() : kGemvSlice;
+    const int bm = path == GTMOE_PATH_BF16 ? mfma_tile_m(T, L->k, L->E) : kGemvSlice;
     // upper bound of the tiles / slices over all groups; without dispatch
     // tables, the shared slices, one row per routed expert and one for every
     // pass of a slice's tokens that an expert could hold beyond its first
@@ -799,6 +799,7 @@ int32_t run_experts(gtmoe_layer *L, int T, int path, hipStream_t s, float *final
         a.desc = w.tile_desc;
         a.out = w.hidden16;
         a.ldo = L->hp;
+        a.bm = bm;
         a.clamp = (float)L->desc.clamp_limit;
         if (L->gate.precision == kFloat32) {  // Float32 experts: their rows' bf16 copies
             a.w0 = L->gate.bf16;
@@ -828,6 +829,7 @@ int32_t run_experts(gtmoe_layer *L, int T, int path, hipStream_t s, float *final
         b.desc = w.tile_desc;
         b.out = w.slot_out;
         b.ldo = L->d;
+        b.bm = bm;
         if (L->down.precision == kFloat32) {
             b.w0 = L->down.bf16;
             b.w_group_stride = (long long)L->down.group_bf16_bytes();
@@ -2117,7 +2119,7 @@ int32_t gtmoe_route_from_logits(gtmoe_layer *L, int32_t tokens, const double *lo
         RUN(ctx, s, "topk", launch_topk(w.logits, T, L->E, L->k, L->balance, w.chosen, w.gates, w.gates32, s));
     }
     RUN(ctx, s, "dispatch",
-        launch_dispatch(w.chosen, T, L->k, L->E, L->S, mfma_tile_m(), w.load, w.offsets, w.rows, w.pos, w.goff,
+        launch_dispatch(w.chosen, T, L->k, L->E, L->S, mfma_tile_m(T, L->k, L->E), w.load, w.offsets, w.rows, w.pos, w.goff,
                         w.tok, w.tile_off, w.tile_desc, w.chunk_cnt, s));
     HIP_TRY(ctx, hipStreamSynchronize(s));
     L->skipped_dispatch = false;

@@ -1,7 +1,7 @@
 // bf16 MFMA grouped GEMM for many tokens per expert (prefill).
 //
-// One workgroup computes a 128-position x 256-column tile of one group
-// (expert) with v_mfma_f32_32x32x16_bf16, fp32 accumulation:
+// One workgroup computes a 128-position (few tokens per expert: 64-position,
+// mfma_tile_m) x 256-column tile of one group (expert) with v_mfma_f32_32x32x16_bf16, fp32 accumulation:
 //   gate/up  A = activations gathered by token (bf16), B = 128 gate rows and
 //            the same 128 up rows of the expert, dequantized (Int8 code or
 //            e2m1 code times its fp32 block scale, rounded to bf16); the
@@ -49,7 +49,6 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int BM = 128;    // positions per tile
 constexpr int BN = 256;    // weight rows per tile (gate/up: 128 neurons x 2)
 constexpr int BK = 64;     // K per pipeline step (4 scale blocks)
 
@@ -171,19 +170,23 @@ __device__ __forceinline__ bf16x8 dequant_half(const BRaw<PREC> &r, int i, int h
     return __builtin_bit_cast(bf16x8, o);
 }
 
-// The output tile in LDS: two halves of 64 rows, one activation buffer each,
-// of 128 bf16 columns, row stride OLD (68 words: the rows m and m + 4 that
+// The output tile in LDS: two halves of BM / 2 rows, one activation buffer
+// each, of 128 bf16 columns, row stride OLD (68 words: the rows m and m + 4 that
 // one ds_write covers fall on disjoint banks).  An activation buffer holds
-// one K step of the tile (128 rows of 128 bytes) or one output half.
+// one K step of the tile (BM rows of 128 bytes) or one output half.
 constexpr int OLD = 136;
-constexpr int kBufBytes = 64 * OLD * 2 > BM * BK * 2 ? 64 * OLD * 2 : BM * BK * 2;
+template <int BM>
+constexpr int buf_bytes()
+{
+    return BM / 2 * OLD * 2 > BM * BK * 2 ? BM / 2 * OLD * 2 : BM * BK * 2;
+}
 
-// Rows [0, M) of the LDS output tile (row m at os[m / 64] + (m % 64) OLD)
+// Rows [0, M) of the LDS output tile (row m at os[m / (BM / 2)] + (m % (BM / 2)) OLD)
 // to out rows p0 + m; tile column c goes to output column col_of(c) (groups
 // of 8 tile columns map to 8 consecutive output columns).  Thread t stores
 // the 16-byte pieces t + 256 i (row piece / 16, columns 8 (piece % 16) ..).
 // Widths or strides that are not multiples of 8 columns take 2-byte stores.
-template <typename ColOf>
+template <int BM, typename ColOf>
 __device__ __forceinline__ void store_tile(const MfmaArgs &a, const uint16_t *os0, const uint16_t *os1, int p0, int M,
                                            ColOf col_of)
 {
@@ -198,13 +201,13 @@ __device__ __forceinline__ void store_tile(const MfmaArgs &a, const uint16_t *os
             const uint16_t *os = i < BM * 8 / 256 ? os0 : os1;  // rows 16 i + tid / 16
             if (m < M && n < a.n)
                 *reinterpret_cast<uint4 *>(out + (size_t)(p0 + m) * a.ldo + n) =
-                    *reinterpret_cast<const uint4 *>(os + (m & 63) * OLD + c);
+                    *reinterpret_cast<const uint4 *>(os + (m & (BM / 2 - 1)) * OLD + c);
         }
     } else {
         for (int e = tid; e < BM * 128; e += 256) {
             const int m = e >> 7, c = e & 127;
             const int n = col_of(c);
-            if (m < M && n < a.n) out[(size_t)(p0 + m) * a.ldo + n] = (m < 64 ? os0 : os1)[(m & 63) * OLD + c];
+            if (m < M && n < a.n) out[(size_t)(p0 + m) * a.ldo + n] = (m < BM / 2 ? os0 : os1)[(m & (BM / 2 - 1)) * OLD + c];
         }
     }
 }
@@ -219,9 +222,9 @@ __device__ __forceinline__ char *pick(char *b0, char *b1, char *b2)
 
 // One tile whose positions lie in its first MI 32-row blocks (M <= 32 MI):
 // the blocks past them are neither loaded nor multiplied.  b0, b1, b2: the
-// three activation buffers (kBufBytes of LDS each, separate arrays, so that
+// three activation buffers (buf_bytes of LDS each, separate arrays, so that
 // the compiler tells their accesses apart).
-template <int PREC, bool GATEUP, int MI>
+template <int PREC, bool GATEUP, int MI, int BM>
 __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1, char *b2, int g, int p0, int M,
                                           int ntile)
 {
@@ -495,8 +498,8 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
     // to half i / 2, LDS column wave * 32 + nn.
     uint16_t *os0 = reinterpret_cast<uint16_t *>(b0), *os1 = reinterpret_cast<uint16_t *>(b1);
     auto put4 = [&](int i, int q, uint32_t lo, uint32_t hi) {  // neurons 8 q + 4 h .. + 3
-        uint16_t *os = i < 2 ? os0 : os1;
-        const int m = (i & 1) * 32 + col;
+        uint16_t *os = 32 * i < BM / 2 ? os0 : os1;
+        const int m = (32 * i) % (BM / 2) + col;
         *reinterpret_cast<uint2 *>(os + m * OLD + wave * 32 + 8 * q + 4 * h) = make_uint2(lo, hi);
     };
     if constexpr (GATEUP) {
@@ -524,7 +527,7 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
         else emit_all(std::false_type{});
         __syncthreads();
         // tile column c is hidden column ntile * 128 + c
-        store_tile(a, os0, os1, p0, M, [&](int c) { return ntile * (BN / 2) + c; });
+        store_tile<BM>(a, os0, os1, p0, M, [&](int c) { return ntile * (BN / 2) + c; });
     } else {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -538,18 +541,18 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
                     put4(i, q, pack_bf16(acc[i][j][r], acc[i][j][r + 1]), pack_bf16(acc[i][j][r + 2], acc[i][j][r + 3]));
                 }
             __syncthreads();
-            store_tile(a, os0, os1, p0, M, [&](int c) { return ntile * BN + (c >> 5) * 64 + j * 32 + (c & 31); });
+            store_tile<BM>(a, os0, os1, p0, M, [&](int c) { return ntile * BN + (c >> 5) * 64 + j * 32 + (c & 31); });
             if (j == 0) __syncthreads();  // the next pass rewrites the LDS tile
         }
     }
 }
 
-template <int PREC, bool GATEUP>
-__global__ __launch_bounds__(256, 2) void mfma_gemm_kernel(MfmaArgs a)
+template <int PREC, bool GATEUP, int BM>
+__global__ __launch_bounds__(256, BM == 64 && PREC == kFP4 ? 3 : 2) void mfma_gemm_kernel(MfmaArgs a)
 {
-    __shared__ __attribute__((aligned(16))) char buf0[kBufBytes];
-    __shared__ __attribute__((aligned(16))) char buf1[kBufBytes];
-    __shared__ __attribute__((aligned(16))) char buf2[kBufBytes];
+    __shared__ __attribute__((aligned(16))) char buf0[buf_bytes<BM>()];
+    __shared__ __attribute__((aligned(16))) char buf1[buf_bytes<BM>()];
+    __shared__ __attribute__((aligned(16))) char buf2[buf_bytes<BM>()];
 
     const int j8 = blockIdx.x >> 3;
     const int ntiles = *a.count;
@@ -562,17 +565,29 @@ __global__ __launch_bounds__(256, 2) void mfma_gemm_kernel(MfmaArgs a)
     const int p0 = dsc.y;  // first position of the tile
     const int M = dsc.z;   // positions in the tile
     // an expert's last tile is usually partly filled: multiply only the
-    // 32-row blocks that hold positions (fewer than three run as two: the
-    // dequantization, the same for any M, then bounds the time anyway)
-    if (M > 96)
-        gemm_tile<PREC, GATEUP, 4>(a, buf0, buf1, buf2, g, p0, M, ntile);
-    else if (M > 64)
-        gemm_tile<PREC, GATEUP, 3>(a, buf0, buf1, buf2, g, p0, M, ntile);
-    else
-        gemm_tile<PREC, GATEUP, 2>(a, buf0, buf1, buf2, g, p0, M, ntile);
+    // 32-row blocks that hold positions (with tiles of 128, fewer than three
+    // run as two: the dequantization, the same for any M, then bounds the time
+    // anyway)
+    if constexpr (BM == 64) {
+        if (M > 32) gemm_tile<PREC, GATEUP, 2, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
+        else gemm_tile<PREC, GATEUP, 1, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
+    } else {
+        if (M > 96) gemm_tile<PREC, GATEUP, 4, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
+        else if (M > 64) gemm_tile<PREC, GATEUP, 3, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
+        else gemm_tile<PREC, GATEUP, 2, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
+    }
 }
 
-int mfma_tile_m() { return BM; }
+// Tiles of 64 positions while the experts average at most 48 routed tokens:
+// most of a 128-position tile would be empty, the smaller tile's registers let
+// FP4 hold three workgroups per CU (two for Int8, whose stages are larger) and
+// a tile of up to 32 positions multiplies one row block.  Layer times with
+// tiles of 128 and 64: d = 2048, h = 1024, 64 + 1 FP4 experts, k = 4: 130
+// tokens 112.5 -> 96.0 us, 333 124.3 -> 109.8, 700 149.6 -> 131.3, 1024 (64 a
+// head) 160.5 -> 156.9, 1500 173.1 against 184.5; d = 1024, h = 2048, 16 Int8
+// experts, k = 2: 128 tokens 59.8 -> 57.5, 300 63.6 against 63.9, 500 (62 a
+// head) 67.5 against 73.8.
+int mfma_tile_m(int T, int k, int E) { return (long long)T * k <= 48LL * E ? 64 : 128; }
 
 // One 16-byte unit of the bf16 copy per thread: fp32 units 2u and 2u + 1 of
 // a row (8 values), rounded as pack_bf16 rounds.  Threads run down the rows
@@ -619,10 +634,16 @@ hipError_t launch_mfma(const MfmaArgs &a, int precision, int max_tiles, hipStrea
     MfmaArgs b = a;
     b.ntiles_n = (a.n + COLS - 1) / COLS;
     const dim3 grid((unsigned)((max_tiles + 7) / 8 * 8 * b.ntiles_n));
+    auto launch = [&](auto prec_tag) {
+        constexpr int P = decltype(prec_tag)::value;
+        if (a.bm == 64) hipLaunchKernelGGL((mfma_gemm_kernel<P, GATEUP, 64>), grid, dim3(256), 0, s, b);
+        else hipLaunchKernelGGL((mfma_gemm_kernel<P, GATEUP, 128>), grid, dim3(256), 0, s, b);
+    };
+    if (a.bm != 64 && a.bm != 128) return hipErrorInvalidValue;
     switch (precision) {
-    case kInt8: hipLaunchKernelGGL((mfma_gemm_kernel<kInt8, GATEUP>), grid, dim3(256), 0, s, b); break;
-    case kFP4: hipLaunchKernelGGL((mfma_gemm_kernel<kFP4, GATEUP>), grid, dim3(256), 0, s, b); break;
-    case kFloat32: hipLaunchKernelGGL((mfma_gemm_kernel<kFloat32, GATEUP>), grid, dim3(256), 0, s, b); break;
+    case kInt8: launch(std::integral_constant<int, kInt8>{}); break;
+    case kFP4: launch(std::integral_constant<int, kFP4>{}); break;
+    case kFloat32: launch(std::integral_constant<int, kFloat32>{}); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

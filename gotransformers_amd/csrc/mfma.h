@@ -27,6 +27,7 @@ struct MfmaArgs {
     const int32_t *count;  // number of m-tiles (the rest of the grid exits)
     const int4 *desc;      // per m-tile: group, first position, positions, 0
     int ntiles_n;          // column tiles (set by the launcher)
+    int bm;                // positions per m-tile (mfma_tile_m)
     void *out;  // bf16: gate/up hidden rows, down slot outputs
     int ldo;
     float clamp;
@@ -36,6 +37,7 @@ struct MfmaArgs {
 hipError_t launch_bf16_rows(const void *rows_f32, void *rows_bf16, int rows_p, int kp, hipStream_t s);
 hipError_t launch_mfma_gateup(const MfmaArgs &a, int precision, int max_tiles, hipStream_t s);
 hipError_t launch_mfma_down(const MfmaArgs &a, int precision, int max_tiles, hipStream_t s);
-int mfma_tile_m();
+// Positions per m-tile, 64 or 128, for T tokens of k choices among E experts.
+int mfma_tile_m(int T, int k, int E);
 
 }  // namespace gtmoe

@@ -321,3 +321,29 @@ def test_bf16_stack_norm_done_by_the_combine(ctx, d, hash_mid):
     e = rel_err(x, ref)
     say(f"[d={d} hash_mid={hash_mid}] max rel err {e:.3e}")
     assert e <= BF16_TOL
+
+
+@pytest.mark.parametrize("prec", [FLOAT32, INT8, FP4])
+@pytest.mark.parametrize("T", [15, 16, 17, 47, 48, 49])
+def test_tiles_of_64_and_128_positions(ctx, prec, T):
+    """Hash routing with consecutive ids fills E = 2 experts (k = 1) with about
+    T/2 rows each and T for the shared expert; with E = 1 the tile rule's limit
+    of 48 tokens per expert lies at T = 48.  Widths that are not multiples of
+    the column tiles or of 8 columns."""
+    say(f"m-tiles T={T} precision {prec}")
+    for E, tokens in ((1, T), (2, 4 * T)):
+        spec = make_moe(gt.encode_rows, d=200, h=301, E=E, k=1, S=1, precision=prec, seed=41 + E, std=0.05,
+                        bias_std=0.02, use_hash=True)
+        rng = np.random.default_rng(T)
+        x = rng.normal(size=(tokens, 200))
+        ids = np.arange(tokens)
+        m = gt.MixtureOfExperts.from_spec(ctx, spec)
+        try:
+            y = m.forward(x, ids, path=gt.PATH_BF16)
+            r = m.last_routing()
+        finally:
+            m.destroy()
+        check_dispatch(r, E)
+        ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates)
+        e = rel_err(y, ref.outputs)
+        assert e <= BF16_TOL, e
