@@ -635,3 +635,28 @@ def test_dispatch_at_the_edges_of_token_waves_and_chunks(ctx, E, k, T):
         assert np.array_equal(g.rows, d.rows)
     ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates)
     assert rel_err(y, ref.outputs) <= 2e-2  # the bf16 path's bar
+
+
+@pytest.mark.parametrize("E,k", [(6, 3), (64, 6), (128, 8), (256, 8)])
+def test_scores_that_share_their_upper_bits(ctx, E, k):
+    """Scores that differ only below the upper 32 bits of the double, or not
+    at all, and infinite balance biases: the choices and gates to the bit."""
+    say(f"top-k close scores E={E} k={k}")
+    rng = np.random.default_rng(E)
+    T = 256
+    logits = 25.0 + 1e-10 * rng.integers(0, 40, size=(T, E))  # affinity sqrt(logit): gaps of 1e-11, and ties
+    logits[64:128] = 25.0 + 1e-10 * np.arange(E)[::-1]
+    logits[128:192] = rng.normal(size=(64, E))
+    bal = np.zeros(E)
+    for b in (bal, np.where(np.arange(E) % 3 == 0, -np.inf, bal), np.where(np.arange(E) % 4 == 1, np.inf, bal),
+              np.full(E, -5.0)):
+        spec = make_moe(gt.encode_rows, d=4, h=4, E=E, k=k, seed=1)
+        m = gt.MixtureOfExperts.from_spec(ctx, spec)
+        try:
+            m.balance_biases = b
+            got = m.route_from_logits(logits)
+        finally:
+            m.destroy()
+        want = oracle.route_from_logits(logits, k, b)
+        assert np.array_equal(got.chosen, want.chosen)
+        assert np.array_equal(got.gates.view(np.int64), want.gates.view(np.int64))
