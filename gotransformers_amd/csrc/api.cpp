@@ -1310,7 +1310,9 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
         const int32_t goff_r[2] = {0, T};
         HIP_TRY(ctx, hipMemcpyAsync(tw.goff_router, goff_r, sizeof goff_r, hipMemcpyHostToDevice, s));
         RUN(ctx, s, "router", launch_router(w.xf, dp, T, d, L->router_w, dp, tw.zero_bias, E, w.logits, s));
-        const LoraArgs ar = lora_args(L->ad_router, T, nullptr, tw.goff_router);
+        rc = upload_outer_tiles(ctx, {0, T}, tw.rt, s);
+        if (rc != GTMOE_OK) return rc;
+        const LoraArgs ar = lora_args(L->ad_router, T, nullptr, tw.goff_router, &tw.rt);
         RUN(ctx, s, "lora_down", launch_lora_down(ar, w.xf, dp, nullptr, tw.u_router, s));
         RUN(ctx, s, "lora_up_bias", launch_lora_up_bias_f64(ar, tw.u_router, w.logits, E, L->router_b, s));
         RUN(ctx, s, "topk", launch_topk(w.logits, T, E, k, L->balance, w.chosen, w.gates, w.gates32, s));
@@ -1338,7 +1340,6 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
     tw.ntiles_tr = (int)ttr.size();
     tw.tile_tr = bt;
     rc = upload_outer_tiles(ctx, goff, tw.ot, s);
-    if (rc == GTMOE_OK) rc = upload_outer_tiles(ctx, {0, T}, tw.rt, s);
     if (rc != GTMOE_OK) return rc;
 
     // the bare products x W^T by the decode GEMV kernels (raw mode, over the
@@ -1374,7 +1375,7 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
         float *pre, *u;
     };
     for (const Role &r : {Role{L->gate, L->ad_gate, tw.gpre, tw.u_gate}, Role{L->up, L->ad_up, tw.upre, tw.u_up}}) {
-        const LoraArgs la = lora_args(r.a, P, tw.pgroup, w.goff);
+        const LoraArgs la = lora_args(r.a, P, tw.pgroup, w.goff, &tw.ot);
         RUN(ctx, s, "lora_down", launch_lora_down(la, w.xf, dp, w.tok, r.u, s));
         RUN(ctx, s, "lora_up_bias", launch_lora_up_bias(la, r.u, r.pre, hp, r.m.biases, s));
     }
@@ -1397,7 +1398,7 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
     b.ld_out = d;
     b.raw = 1;
     RUN(ctx, s, "gemv_down", launch_gemv_down(b, L->down.precision, slices, s));
-    const LoraArgs ld = lora_args(L->ad_down, P, tw.pgroup, w.goff);
+    const LoraArgs ld = lora_args(L->ad_down, P, tw.pgroup, w.goff, &tw.ot);
     RUN(ctx, s, "lora_down", launch_lora_down(ld, w.hidden32, hp, nullptr, tw.u_down, s));
     RUN(ctx, s, "lora_up_bias", launch_lora_up_bias(ld, tw.u_down, w.slot_out, d, L->down.biases, s));
     RUN(ctx, s, "combine",

@@ -330,71 +330,159 @@ __global__ __launch_bounds__(256) void sum_chunks_kernel(const float *__restrict
     out[o] = s;
 }
 
-__device__ __forceinline__ float wave_sum(float v)
-{
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
+// The adapters' two projections onto the ranks, as fp32 16x16x4 MFMAs over
+// the position tiles of one group (LoraArgs::otiles):
+//   u[p][j] = sum_i in[row(p)][i] * A[g][j][i]                  (TO_RANK = down)
+//   t[p][j] = scale[g] * sum_n grad[p][n] * B[g][n][j]           (TO_RANK = back)
+// A workgroup takes 16 positions of a tile (blockIdx.z) and 16 ranks, its four
+// waves a quarter of the sum each, in steps of 16 values: a lane reads four
+// consecutive values of its position (and of its rank's row of A, or its
+// rank's column of four rows of B), the four k of four MFMAs.  The waves' sums
+// are added in wave order through LDS.  The loads' latency bounds it, so eight
+// steps are in flight.  (One wave per (position, rank), or one workgroup per
+// position, read the adapter's values for every position: 3584 positions, 16
+// ranks, 512 to 1024 values 17.4 and 16.1 us per launch, now 8.4 and
+// 6.4.)
+constexpr int kOpPositions = 64;  // positions of a tile at most
+constexpr int kRkPositions = 16;  // positions of a workgroup
+constexpr int kRkStep = 16;       // values per step
+constexpr int kRkDepth = 8;       // steps in flight
 
-// u[p][j] = sum_i in[row(p)][i] * A[g(p)][j][i]; one wave per (position,
-// rank j).  Rows are read as float4 runs over the padded width kin (zeros
-// past the width in both operands); the loads are unconditional (clamped
-// index, masked sum) so the compiler keeps them all in flight.
-__global__ __launch_bounds__(256) void lora_down_kernel(LoraArgs a, const float *__restrict__ in, int ld_in,
-                                                        const int32_t *__restrict__ in_tok, float *__restrict__ u)
+template <bool BACK>
+__global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const float *__restrict__ in, int ld_in,
+                                                           const int32_t *__restrict__ in_tok, float *__restrict__ out)
 {
+    __shared__ float red[4][4][64];
+    const int4 td = a.otiles[blockIdx.x];
+    const int g = td.x, p0 = td.y + kRkPositions * blockIdx.z, m = td.z - kRkPositions * (int)blockIdx.z;
+    if (m <= 0) return;  // workgroup-uniform
     const int lane = threadIdx.x & 63;
-    const int wv = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wv >= a.P * a.R) return;  // wave-uniform
-    const int p = wv / a.R, j = wv - p * a.R;
-    const int g = a.pgroup ? a.pgroup[p] : 0;
-    const int row = in_tok ? in_tok[p] : p;
-    const float4 *x = reinterpret_cast<const float4 *>(in + (size_t)row * ld_in);
-    const float4 *A = reinterpret_cast<const float4 *>(a.A + ((size_t)g * a.R + j) * a.kin);
-    const int n4 = a.kin / 4;
-    float s = 0.f;
-#pragma unroll 4
-    for (int i = lane; i < n4 + 63; i += 64) {
-        const int c = min(i, n4 - 1);
-        const float4 xv = x[c], av = A[c];
-        const float d = xv.x * av.x + xv.y * av.y + xv.z * av.z + xv.w * av.w;
-        s += i < n4 ? d : 0.f;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, kg = lane >> 4;
+    const int j = blockIdx.y * 16 + li, jc = min(j, a.R - 1);
+    const int nval = BACK ? a.rows : a.kin;
+    const bool vec = (ld_in & 3) == 0;  // BACK over output gradients: rows of any width
+    const int p = p0 + min(li, m - 1);
+    const float *row = in + (size_t)(in_tok ? in_tok[p] : p) * ld_in;
+    const float *ad = BACK ? a.B + (size_t)g * a.rows * a.R + jc : a.A + ((size_t)g * a.R + jc) * a.kin;
+    const int steps = (nval + kRkStep - 1) / kRkStep;
+    const int s0 = wave * steps / 4, s1 = (wave + 1) * steps / 4;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int sb = s0; sb < s1; sb += kRkDepth) {
+        f32x4 x[kRkDepth], w[kRkDepth];
+#pragma unroll
+        for (int q = 0; q < kRkDepth; ++q) {
+            // steps past the wave's last repeat it and are not multiplied
+            const int n = kRkStep * min(sb + q, s1 - 1) + 4 * kg;
+            if constexpr (BACK) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[q][e] = ad[(size_t)min(n + e, nval - 1) * a.R];
+                if (vec && nval % kRkStep == 0) {  // uniform
+                    x[q] = *reinterpret_cast<const f32x4 *>(row + n);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float v = row[min(n + e, nval - 1)];
+                        x[q][e] = n + e < nval ? v : 0.f;
+                    }
+                }
+            } else {  // padded rows of kin values, a multiple of 64
+                w[q] = *reinterpret_cast<const f32x4 *>(ad + n);
+                x[q] = *reinterpret_cast<const f32x4 *>(row + n);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kRkDepth; ++q) {
+            if (sb + q >= s1) break;  // wave-uniform
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q][e], w[q][e], acc, 0, 0, 0);
+        }
     }
-    s = wave_sum(s);
-    if (lane == 0) u[(size_t)p * a.R + j] = s;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave][v][lane] = acc[v];
+    __syncthreads();
+    // register v of lane l: position 4 (l / 16) + v, rank l % 16; wave w
+    // finishes register w
+    const int q = 4 * kg + wave;
+    if (j >= a.R || q >= m) return;
+    const float s = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
+    out[(size_t)(p0 + q) * a.R + j] = BACK ? a.scale[g] * s : s;
 }
 
-// out[p][n] = (out[p][n] + scale[g] * sum_j B[g][n][j] u[p][j]) + bias[n]
-// for n < rows (the reference adds the adapter, then the bias).
+// The ranks' two projections back, over the position tiles of one group:
+//   out[p][n] = (out[p][n] + scale[g] * sum_j B[g][n][j] u[p][j]) + bias[n], n < rows
+// (the reference adds the adapter, then the bias), and lora_dx_kernel's
+//   dx[p][i] += sum_j t[p][j] * A[g][j][i], i < width.
+// A thread keeps its row of B (its column of A) for up to 16 positions of the
+// tile, eight of them in flight (before, a position at a time: 16-20 and 17 us
+// per launch over 3584 positions, 512 to 1024 columns, 16 ranks; 7.6 and
+// 7.4 as here, where the rows' read and write take 3 to 6).
+constexpr int kFromRank = 16;  // positions per thread
+
+// The first 16 ranks of m <= kFromRank positions in LDS, zero past the rank
+// (read back as broadcasts: scalar loads came one position at a time).
+__device__ __forceinline__ void stage_ranks(f32x4 (&us)[kFromRank][4], const float *__restrict__ u, int m, int R)
+{
+    const int q = threadIdx.x >> 4, j = threadIdx.x & 15;
+    const float v = u[(size_t)min(q, m - 1) * R + min(j, R - 1)];
+    reinterpret_cast<float *>(us)[threadIdx.x] = j < R ? v : 0.f;
+    __syncthreads();
+}
+
+__device__ __forceinline__ float rank_dot(const f32x4 (&u)[4], const float (&c)[16])
+{
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s = fmaf(c[j], u[j >> 2][j & 3], s);  // both zero past the rank
+    return s;
+}
+
 template <typename OutT>
 __global__ __launch_bounds__(256) void lora_up_bias_kernel(LoraArgs a, const float *__restrict__ u,
                                                            OutT *__restrict__ out, int ld_out,
                                                            const float *__restrict__ bias32,
                                                            const double *__restrict__ bias64)
 {
+    __shared__ f32x4 us[kFromRank][4];
+    const int4 td = a.otiles[blockIdx.y];
+    const int g = td.x, q0 = blockIdx.z * kFromRank, q1 = min(td.z, q0 + kFromRank);
+    if (q0 >= q1) return;  // workgroup-uniform
     const int n = blockIdx.x * 256 + threadIdx.x;
-    const int p = blockIdx.y;
+    stage_ranks(us, u + (size_t)(td.y + q0) * a.R, q1 - q0, a.R);
     if (n >= a.rows) return;
-    const int g = a.pgroup ? a.pgroup[p] : 0;
     const float *B = a.B + ((size_t)g * a.rows + n) * a.R;
-    const float *up = u + (size_t)p * a.R;
-    float s = 0.f;
-    if ((a.R & 3) == 0) {  // the row's ranks as float4 runs (rows are 16-byte aligned)
-        for (int j = 0; j < a.R; j += 4) {
-            const float4 b4 = *reinterpret_cast<const float4 *>(B + j);
-            s = fmaf(b4.x, up[j], s);
-            s = fmaf(b4.y, up[j + 1], s);
-            s = fmaf(b4.z, up[j + 2], s);
-            s = fmaf(b4.w, up[j + 3], s);
+    float bc[16];
+    if ((a.R & 3) == 0) {  // rows are 16-byte aligned
+#pragma unroll
+        for (int j = 0; j < 16; j += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(B + min(j, a.R - 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bc[j + e] = j < a.R ? v[e] : 0.f;
         }
     } else {
-        for (int j = 0; j < a.R; ++j) s = fmaf(B[j], up[j], s);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const float v = B[min(j, a.R - 1)];
+            bc[j] = j < a.R ? v : 0.f;
+        }
     }
-    OutT &o = out[(size_t)p * ld_out + n];
-    if constexpr (sizeof(OutT) == 8) {
-        o = (o + (double)(a.scale[g] * s)) + bias64[n];
-    } else {
-        o = (o + a.scale[g] * s) + bias32[(size_t)g * a.rows + n];
+    const float sc = a.scale[g];
+    OutT bias;
+    if constexpr (sizeof(OutT) == 8) bias = bias64[n];
+    else bias = bias32[(size_t)g * a.rows + n];
+    for (int q = q0; q < q1; q += 8) {
+        OutT o[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = out[(size_t)(td.y + min(q + i, q1 - 1)) * ld_out + n];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (q + i >= q1) break;
+            const int p = td.y + q + i;
+            const float *up = u + (size_t)p * a.R;
+            float s = rank_dot(us[q + i - q0], bc);
+            for (int j = 16; j < a.R; ++j) s = fmaf(B[j], up[j], s);
+            out[(size_t)p * ld_out + n] = (o[i] + (OutT)(sc * s)) + bias;
+        }
     }
 }
 
@@ -412,7 +500,6 @@ __global__ __launch_bounds__(256) void lora_up_bias_kernel(LoraArgs a, const flo
 // directly (each output has one writer); the tiles of larger groups write
 // partial[tile][j][c] and lora_tiles_sum_kernel adds them in tile order, in
 // float64, to the accumulator.
-constexpr int kOpPositions = 64;
 
 struct OuterArgs {
     const int4 *tiles;
@@ -522,87 +609,36 @@ void launch_outer(OuterArgs o, const LoraArgs &a, float *scratch, hipStream_t s)
                            a.otoff, a.omulti);
 }
 
-// t[p][j] = scale[g] * sum_n grad[p][n] * B[g][n][j]; one workgroup per
-// position and 16 ranks: lane l of wave w takes rows n = 64 (4 i + w) + l,
-// reading the gradient once and each row's 16 ranks of B as contiguous
-// float4 runs; each wave adds its lanes' partial sums, and the four waves'
-// sums are added in wave order through LDS.
-constexpr int kTRanks = 16;
-
-__global__ __launch_bounds__(256) void lora_t_kernel(LoraArgs a, const float *__restrict__ grad, int ld_g,
-                                                     float *__restrict__ t)
-{
-    __shared__ float part[4][kTRanks];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nj = (a.R + kTRanks - 1) / kTRanks;
-    const int p = blockIdx.x / nj, j0 = (blockIdx.x - p * nj) * kTRanks;
-    const int g = a.pgroup ? a.pgroup[p] : 0;
-    const float *gr = grad + (size_t)p * ld_g;
-    const float *B = a.B + (size_t)g * a.rows * a.R;
-    const bool vec = (a.R & 3) == 0 && j0 + kTRanks <= a.R;
-    float s[kTRanks];
-#pragma unroll
-    for (int j = 0; j < kTRanks; ++j) s[j] = 0.f;
-#pragma unroll 2
-    for (int n = 64 * wave + lane; n < a.rows; n += 256) {
-        const float gv = gr[n];
-        const float *br = B + (size_t)n * a.R + j0;
-        if (vec) {
-#pragma unroll
-            for (int q = 0; q < kTRanks / 4; ++q) {
-                const float4 b4 = *reinterpret_cast<const float4 *>(br + 4 * q);
-                s[4 * q] = fmaf(gv, b4.x, s[4 * q]);
-                s[4 * q + 1] = fmaf(gv, b4.y, s[4 * q + 1]);
-                s[4 * q + 2] = fmaf(gv, b4.z, s[4 * q + 2]);
-                s[4 * q + 3] = fmaf(gv, b4.w, s[4 * q + 3]);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < kTRanks; ++j)
-                if (j0 + j < a.R) s[j] = fmaf(gv, br[j], s[j]);
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kTRanks; ++j) s[j] = wave_sum(s[j]);
-    if (lane < kTRanks) {
-        float v = s[0];
-#pragma unroll
-        for (int j = 1; j < kTRanks; ++j)
-            if (lane == j) v = s[j];
-        part[wave][lane] = v;
-    }
-    __syncthreads();
-    if (wave == 0 && lane < kTRanks && j0 + lane < a.R)
-        t[(size_t)p * a.R + j0 + lane] = a.scale[g] * (((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane]);
-}
-
-// dx[p][i] += sum_j t[p][j] * A[g][j][i], i < width; thread i takes
-// positions pp blockIdx.y .. + pp - 1 and keeps its column of A (up to 16
-// ranks) in registers while the group stays the same (pp = 8 when there are
-// positions enough to fill the GPU that way, else 1).
 __global__ __launch_bounds__(256) void lora_dx_kernel(LoraArgs a, const float *__restrict__ t,
-                                                      float *__restrict__ dx, int ld_dx, int pp)
+                                                      float *__restrict__ dx, int ld_dx)
 {
+    __shared__ f32x4 ts[kFromRank][4];
+    const int4 td = a.otiles[blockIdx.y];
+    const int g = td.x, q0 = blockIdx.z * kFromRank, q1 = min(td.z, q0 + kFromRank);
+    if (q0 >= q1) return;  // workgroup-uniform
     const int i = blockIdx.x * 256 + threadIdx.x;
+    stage_ranks(ts, t + (size_t)(td.y + q0) * a.R, q1 - q0, a.R);
     if (i >= a.width) return;
-    const int pb = blockIdx.y * pp, pe = min(a.P, pb + pp);
-    int gcur = -1;
+    const float *A = a.A + (size_t)g * a.R * a.kin + i;
     float ac[16];
-    for (int p = pb; p < pe; ++p) {
-        const int g = a.pgroup ? a.pgroup[p] : 0;
-        const float *A = a.A + (size_t)g * a.R * a.kin + i;
-        if (g != gcur) {  // uniform
 #pragma unroll
-            for (int j = 0; j < 16; ++j) ac[j] = A[(size_t)min(j, a.R - 1) * a.kin];  // in bounds; j >= R unused
-            gcur = g;
+    for (int j = 0; j < 16; ++j) {
+        const float v = A[(size_t)min(j, a.R - 1) * a.kin];
+        ac[j] = j < a.R ? v : 0.f;
+    }
+    for (int q = q0; q < q1; q += 8) {
+        float o[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) o[r] = dx[(size_t)(td.y + min(q + r, q1 - 1)) * ld_dx + i];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            if (q + r >= q1) break;
+            const int p = td.y + q + r;
+            const float *tp = t + (size_t)p * a.R;
+            float s = rank_dot(ts[q + r - q0], ac);
+            for (int j = 16; j < a.R; ++j) s = fmaf(tp[j], A[(size_t)j * a.kin], s);
+            dx[(size_t)p * ld_dx + i] = o[r] + s;
         }
-        const float *tp = t + (size_t)p * a.R;
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-            if (j < a.R) s = fmaf(tp[j], ac[j], s);
-        for (int j = 16; j < a.R; ++j) s = fmaf(tp[j], A[(size_t)j * a.kin], s);
-        dx[(size_t)p * ld_dx + i] += s;
     }
 }
 
@@ -676,15 +712,16 @@ __global__ __launch_bounds__(256) void expert_output_grad_kernel(const double *_
                                                                  const double *__restrict__ gates,
                                                                  float *__restrict__ eg)
 {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    const int p = blockIdx.y;
-    if (i >= ld) return;
+    // a workgroup takes a position's whole row: its token, group and gate are
+    // looked up once
+    const int p = blockIdx.x;
     const int t = tok[p], g = pgroup[p];
     double w = 1.0;
     if (g >= S)
         for (int j = 0; j < k; ++j)
             if (chosen[(size_t)t * k + j] == g - S) w = gates[(size_t)t * k + j];
-    eg[(size_t)p * ld + i] = i < d ? (float)(og[(size_t)t * d + i] * w) : 0.f;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < ld; i += 256) eg[(size_t)p * ld + i] = i < d ? (float)(og[(size_t)t * d + i] * w) : 0.f;
 }
 
 // Input gradient of each token: the shared experts' rows, then its routed
@@ -720,7 +757,10 @@ __global__ __launch_bounds__(256) void router_input_grad_kernel(const float *__r
     const int t = blockIdx.y;
     if (i >= d) return;
     float s = 0.f;
-    for (int e = 0; e < E; ++e) s = fmaf(lg[(size_t)t * E + e], w[(size_t)e * ldw + i], s);
+    for (int e = 0; e < E; ++e) {
+        const float l = lg[(size_t)t * E + e];
+        if (l != 0.f) s = fmaf(l, w[(size_t)e * ldw + i], s);  // uniform: zero but for the chosen experts
+    }
     dx[(size_t)t * ld_dx + i] = s;
 }
 
@@ -795,12 +835,21 @@ int rows_transposed_colblocks(int nblocks, int tile)
     return tile == kMtPositions ? (nblocks + kMtBlocks - 1) / kMtBlocks : (nblocks + 63) / 64;
 }
 
+namespace {
+bool tiles_given(const LoraArgs &a) { return a.notiles > 0 && a.otiles && a.otoff; }
+dim3 from_rank_grid(const LoraArgs &a, int columns)
+{
+    return dim3((columns + 255) / 256, a.notiles, kOpPositions / kFromRank);
+}
+}  // namespace
+
 hipError_t launch_lora_down(const LoraArgs &a, const float *in, int ld_in, const int32_t *in_tok, float *u,
                             hipStream_t s)
 {
     if (a.P <= 0 || a.R <= 0) return hipSuccess;
-    const int waves = a.P * a.R;
-    hipLaunchKernelGGL(lora_down_kernel, dim3((waves + 3) / 4), dim3(256), 0, s, a, in, ld_in, in_tok, u);
+    if (!tiles_given(a)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(lora_to_rank_kernel<false>, dim3(a.notiles, (a.R + 15) / 16, kOpPositions / kRkPositions), dim3(256), 0, s, a, in, ld_in,
+                       in_tok, u);
     return hipGetLastError();
 }
 
@@ -808,7 +857,8 @@ hipError_t launch_lora_up_bias(const LoraArgs &a, const float *u, float *out, in
                                hipStream_t s)
 {
     if (a.P <= 0) return hipSuccess;
-    hipLaunchKernelGGL(lora_up_bias_kernel<float>, cols_grid(a.rows, a.P), dim3(256), 0, s, a, u, out, ld_out, bias,
+    if (!tiles_given(a)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(lora_up_bias_kernel<float>, from_rank_grid(a, a.rows), dim3(256), 0, s, a, u, out, ld_out, bias,
                        nullptr);
     return hipGetLastError();
 }
@@ -817,7 +867,8 @@ hipError_t launch_lora_up_bias_f64(const LoraArgs &a, const float *u, double *ou
                                    hipStream_t s)
 {
     if (a.P <= 0) return hipSuccess;
-    hipLaunchKernelGGL(lora_up_bias_kernel<double>, cols_grid(a.rows, a.P), dim3(256), 0, s, a, u, out, ld_out,
+    if (!tiles_given(a)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(lora_up_bias_kernel<double>, from_rank_grid(a, a.rows), dim3(256), 0, s, a, u, out, ld_out,
                        nullptr, bias);
     return hipGetLastError();
 }
@@ -827,20 +878,18 @@ hipError_t launch_lora_backward(const LoraArgs &a, const float *grad, int ld_g, 
                                 double *dB, float *scratch, hipStream_t s)
 {
     if (a.P <= 0 || a.R <= 0) return hipSuccess;
-    if (a.notiles <= 0 || !a.otiles || !a.otoff || (a.nomulti > 0 && (!a.omulti || !scratch)))
-        return hipErrorInvalidValue;
+    if (!tiles_given(a) || (a.nomulti > 0 && (!a.omulti || !scratch))) return hipErrorInvalidValue;
     // dB += scale grad^T u: columns are B's rows n, the sums land at dB[g][n][j]
     launch_outer(OuterArgs{a.otiles, u, a.R, grad, ld_g, nullptr, a.rows, nullptr, a.scale, dB,
                            (long long)a.rows * a.R, 1LL, (long long)a.R},
                  a, scratch, s);
-    hipLaunchKernelGGL(lora_t_kernel, dim3(a.P * ((a.R + kTRanks - 1) / kTRanks)), dim3(256), 0, s, a, grad, ld_g, t);
+    hipLaunchKernelGGL(lora_to_rank_kernel<true>, dim3(a.notiles, (a.R + 15) / 16, kOpPositions / kRkPositions), dim3(256), 0, s, a, grad, ld_g,
+                       nullptr, t);
     // dA += t^T in: columns are the inputs i, the sums land at dA[g][j][i]
     launch_outer(OuterArgs{a.otiles, t, a.R, in, ld_in, in_tok, a.width, nullptr, nullptr, dA, (long long)a.R * a.kin,
                            (long long)a.kin, 1LL},
                  a, scratch, s);
-    const int pp = (long long)((a.width + 255) / 256) * (a.P / 8) >= 1024 ? 8 : 1;
-    hipLaunchKernelGGL(lora_dx_kernel, dim3((a.width + 255) / 256, (a.P + pp - 1) / pp), dim3(256), 0, s, a, t, dx,
-                       ld_dx, pp);
+    hipLaunchKernelGGL(lora_dx_kernel, from_rank_grid(a, a.width), dim3(256), 0, s, a, t, dx, ld_dx);
     return hipGetLastError();
 }
 
@@ -866,7 +915,7 @@ hipError_t launch_expert_output_grad(const double *og, int d, int ld, const int3
                                      float *eg, hipStream_t s)
 {
     if (P <= 0) return hipSuccess;
-    hipLaunchKernelGGL(expert_output_grad_kernel, cols_grid(ld, P), dim3(256), 0, s, og, d, ld, tok, pgroup, S, T, k,
+    hipLaunchKernelGGL(expert_output_grad_kernel, dim3(P), dim3(256), 0, s, og, d, ld, tok, pgroup, S, T, k,
                        chosen, gates, eg);
     return hipGetLastError();
 }

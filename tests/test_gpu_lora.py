@@ -181,3 +181,38 @@ def test_adapter_errors_mirror_the_reference(ctx):
         assert info.value.code == gt.ERR_UNSUPPORTED
     finally:
         m.destroy()
+
+
+@pytest.mark.parametrize("rank", [3, 16, 17, 20])
+@pytest.mark.parametrize("T", [1, 15, 17, 63, 65, 130])
+def test_rank_projections_at_the_edges_of_their_tiles(ctx, T, rank):
+    """Hash routing with one expert (T positions in its group and T in the
+    shared expert's) and the router's T tokens: blocks of 16 positions and tiles
+    of 64, partly filled; ranks below, at and past 16; output-gradient rows 37
+    floats apart, hidden widths that are not multiples of 16."""
+    d, h = 37, 53
+    say(f"rank projections T={T} rank={rank}")
+    spec = make_moe(gt.encode_rows, d=d, h=h, E=1, k=1, S=1, precision=INT8, seed=51, std=0.1, router_std=0.1,
+                    bias_std=0.02)
+    rng = np.random.default_rng(52 + T)
+    alpha = 2.0 * rank
+    adapters = lora.make_adapters(spec, rank, alpha, rng, up_scale=0.05)
+    x = rng.uniform(-1, 1, (T, d))
+    G = rng.uniform(-1, 1, (T, d))
+    m = with_adapters(ctx, spec, adapters, rank, alpha)
+    try:
+        y = m.forward(x)
+        r = m.last_routing()
+        dx = m.backward(G)
+        grads = {key: m.adapter_gradients(*key) for key in keys_of(spec)}
+    finally:
+        m.destroy()
+    ref_y, st = lora.forward(spec, adapters, x, None, chosen=r.chosen)
+    ref_grads = lora.zero_grads(spec, adapters)
+    ref_dx = lora.backward(spec, adapters, st, G, ref_grads)
+    assert rel_err(y, ref_y) <= FWD_TOL
+    assert rel_err(dx, ref_dx) <= GRAD_TOL
+    for key in keys_of(spec):
+        for got, want in zip(grads[key], ref_grads[key]):
+            if np.any(want):
+                assert rel_err(got, want) <= GRAD_TOL, key
