@@ -259,6 +259,8 @@ struct TrainWorkspace {
     double *lg = nullptr;    // [T][E]
     float *lgf = nullptr;    // [T][E]
     float *dxr = nullptr;    // [T][dp]
+    // tables the host makes during a forward, one after the other in `tables`
+    char *tables = nullptr;
     int32_t *pgroup = nullptr;  // [P]
     int4 *tiles_tr = nullptr;  // [P + G]
     int32_t *goff_router = nullptr;  // {0, T}
@@ -272,8 +274,6 @@ struct TrainWorkspace {
         int32_t *toff = nullptr;   // [G + 1] first tile of every group
         int32_t *multi = nullptr;  // [G] groups of more than one tile
         int n = 0, nmulti = 0;
-        std::vector<int4> host_tiles;  // sources of the uploads
-        std::vector<int32_t> host_toff, host_multi;
     } ot, rt;
     float *outer = nullptr;  // [P/64 + G][R][max(dp, hp, E)] tile sums of the adapter gradients
     int P = 0, ntiles_tr = 0, tile_tr = 4;
@@ -1151,6 +1151,15 @@ AdapterSet *adapter_of(gtmoe_layer *L, int role, int index, int *group)
     return which == 0 ? &L->ad_gate : which == 1 ? &L->ad_up : &L->ad_down;
 }
 
+// Bytes of TrainWorkspace::tables: every table of a forward of `cap` tokens,
+// each rounded up to 64 bytes.
+size_t train_tables_bytes(const gtmoe_layer *L, int cap)
+{
+    const size_t P = (size_t)cap * (L->S + L->k), G = L->G, n = lora_outer_tile_positions();
+    return 4 * P + 16 * (P + G) + (16 * (P / n + G) + 4 * (G + 1) + 4 * G) + (16 * ((size_t)cap / n + 1) + 4 * 2 + 4) +
+           4 * 2 + 9 * 64;
+}
+
 int32_t ensure_train_workspace(gtmoe_layer *L, int T)
 {
     TrainWorkspace &tw = L->tw;
@@ -1183,13 +1192,8 @@ int32_t ensure_train_workspace(gtmoe_layer *L, int T)
              [&] { return get(tw.dxu, P * dp); }, [&] { return get(tw.t, std::max(P, (size_t)cap) * R); },
              [&] { return get(tw.dx, (size_t)cap * d); }, [&] { return get(tw.lg, (size_t)cap * E); },
              [&] { return get(tw.lgf, (size_t)cap * E); }, [&] { return get(tw.dxr, (size_t)cap * dp); },
-             [&] { return get(tw.pgroup, P); }, [&] { return get(tw.tiles_tr, P + L->G); },
-             [&] { return get(tw.goff_router, (size_t)2); }, [&] { return get(tw.zero_bias, E); },
+             [&] { return get(tw.tables, train_tables_bytes(L, cap)); }, [&] { return get(tw.zero_bias, E); },
              [&] { return get(tw.partial, (size_t)tw.chunks * P * std::max(hp, dp)); },
-             [&] { return get(tw.ot.tiles, P / lora_outer_tile_positions() + L->G); },
-             [&] { return get(tw.ot.toff, (size_t)L->G + 1); }, [&] { return get(tw.ot.multi, (size_t)L->G); },
-             [&] { return get(tw.rt.tiles, (size_t)cap / lora_outer_tile_positions() + 1); },
-             [&] { return get(tw.rt.toff, (size_t)2); }, [&] { return get(tw.rt.multi, (size_t)1); },
              [&] { return get(tw.outer, (P / lora_outer_tile_positions() + L->G) * R * std::max({hp, dp, E})); }}) {
         rc = step();
         if (rc != GTMOE_OK) {
@@ -1250,31 +1254,47 @@ RowsArgs rows_args(const DeviceMatrix &m, const float *in, int ld_in, const int3
     return r;
 }
 
+// The tables of one adapter forward: written to pinned staging, copied to
+// the same offsets of the device block.
+struct TableWriter {
+    char *host, *dev;
+    size_t off = 0, sent = 0;
+    template <class T>
+    T *put(const std::vector<T> &v)
+    {
+        if (!v.empty()) memcpy(host + off, v.data(), v.size() * sizeof(T));
+        T *p = reinterpret_cast<T *>(dev + off);
+        off = align_up(off + v.size() * sizeof(T), 64);
+        return p;
+    }
+    // everything put since the last send, in one copy
+    hipError_t send(hipStream_t s)
+    {
+        const size_t a = sent;
+        sent = off;
+        return off > a ? hipMemcpyAsync(dev + a, host + a, off - a, hipMemcpyHostToDevice, s) : hipSuccess;
+    }
+};
+
 // Tiles of the adapter gradients over groups whose positions start at goff
-// (goff.size() - 1 groups), uploaded to `ot` (the host copies stay alive
-// until the stream has read them: the caller synchronizes before returning).
-int32_t upload_outer_tiles(gtmoe_context *ctx, const std::vector<int32_t> &goff, TrainWorkspace::OuterTiles &ot,
-                           hipStream_t s)
+// (goff.size() - 1 groups).
+void put_outer_tiles(TableWriter &tables, const std::vector<int32_t> &goff, TrainWorkspace::OuterTiles &ot)
 {
     const int G = (int)goff.size() - 1, n = lora_outer_tile_positions();
-    ot.host_tiles.clear();
-    ot.host_toff.assign(G + 1, 0);
-    ot.host_multi.clear();
+    std::vector<int4> tiles;
+    std::vector<int32_t> toff(G + 1, 0), multi;
     for (int g = 0; g < G; ++g) {
-        ot.host_toff[g] = (int32_t)ot.host_tiles.size();
+        toff[g] = (int32_t)tiles.size();
         const int many = goff[g + 1] - goff[g] > n ? 1 : 0;
-        if (many) ot.host_multi.push_back(g);
-        for (int p = goff[g]; p < goff[g + 1]; p += n)
-            ot.host_tiles.push_back(make_int4(g, p, std::min(n, goff[g + 1] - p), many));
+        if (many) multi.push_back(g);
+        for (int p = goff[g]; p < goff[g + 1]; p += n) tiles.push_back(make_int4(g, p, std::min(n, goff[g + 1] - p), many));
     }
-    ot.host_toff[G] = (int32_t)ot.host_tiles.size();
-    ot.n = (int)ot.host_tiles.size();
-    ot.nmulti = (int)ot.host_multi.size();
-    HIP_TRY(ctx, hipMemcpyAsync(ot.tiles, ot.host_tiles.data(), sizeof(int4) * ot.n, hipMemcpyHostToDevice, s));
-    HIP_TRY(ctx, hipMemcpyAsync(ot.toff, ot.host_toff.data(), sizeof(int32_t) * (G + 1), hipMemcpyHostToDevice, s));
-    if (ot.nmulti)
-        HIP_TRY(ctx, hipMemcpyAsync(ot.multi, ot.host_multi.data(), sizeof(int32_t) * ot.nmulti, hipMemcpyHostToDevice, s));
-    return GTMOE_OK;
+    toff[G] = (int32_t)tiles.size();
+    ot.n = (int)tiles.size();
+    ot.nmulti = (int)multi.size();
+    ot.tiles = tables.put(tiles);
+    ot.toff = tables.put(toff);
+    ot.multi = tables.put(multi);
 }
 
 // Row chunks for the transposed product over `rows` rows: enough four-wave
@@ -1301,17 +1321,27 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
     TrainWorkspace &tw = L->tw;
     const int d = L->d, dp = L->dp, hp = L->hp, E = L->E, S = L->S, k = L->k, G = L->G;
     const bool hash = L->desc.use_hash_routing != 0;
-    HIP_TRY(ctx, hipMemcpyAsync(w.x64, inputs, sizeof(double) * T * d, hipMemcpyHostToDevice, s));
+    // The rows cross the bus as fp32 through pinned staging, as in a forward
+    // without adapters: rounded here as the first kernel would round them, and
+    // the combine's fp32 sums widened here.  Behind them in the staging: the
+    // groups' first positions, and the tables made from them.
+    const size_t nvals = (size_t)T * d, rows_bytes = align_up(sizeof(float) * nvals, 64);
+    const size_t goff_bytes = align_up(sizeof(int32_t) * (G + 1), 64);
+    rc = ensure_stage(L, 2 * rows_bytes + goff_bytes + train_tables_bytes(L, T));
+    if (rc != GTMOE_OK) return rc;
+    TableWriter tables{L->stage + 2 * rows_bytes + goff_bytes, tw.tables};
+    float *hx = reinterpret_cast<float *>(L->stage);
+    for (size_t i = 0; i < nvals; ++i) hx[i] = (float)inputs[i];
     if (hash) HIP_TRY(ctx, hipMemcpyAsync(w.ids, token_ids, sizeof(int64_t) * T, hipMemcpyHostToDevice, s));
-    RUN(ctx, s, "convert_inputs", launch_convert_inputs_f64(w.x64, T, d, w.xf, dp, nullptr, dp, s));
+    RUN(ctx, s, "convert_inputs",
+        launch_convert_inputs_f32(reinterpret_cast<const float *>(L->stage_dev), T, d, w.xf, dp, nullptr, dp, s));
     if (hash) {
         RUN(ctx, s, "hash_route", launch_hash_route(w.ids, T, E, k, w.chosen, w.gates, w.gates32, s));
     } else {
-        const int32_t goff_r[2] = {0, T};
-        HIP_TRY(ctx, hipMemcpyAsync(tw.goff_router, goff_r, sizeof goff_r, hipMemcpyHostToDevice, s));
+        tw.goff_router = tables.put(std::vector<int32_t>{0, T});
+        put_outer_tiles(tables, {0, T}, tw.rt);
+        HIP_TRY(ctx, tables.send(s));
         RUN(ctx, s, "router", launch_router(w.xf, dp, T, d, L->router_w, dp, tw.zero_bias, E, w.logits, s));
-        rc = upload_outer_tiles(ctx, {0, T}, tw.rt, s);
-        if (rc != GTMOE_OK) return rc;
         const LoraArgs ar = lora_args(L->ad_router, T, nullptr, tw.goff_router, &tw.rt);
         RUN(ctx, s, "lora_down", launch_lora_down(ar, w.xf, dp, nullptr, tw.u_router, s));
         RUN(ctx, s, "lora_up_bias", launch_lora_up_bias_f64(ar, tw.u_router, w.logits, E, L->router_b, s));
@@ -1323,8 +1353,16 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
                         w.tile_off, w.tile_desc, w.chunk_cnt, s));
     // positions of every group, and work tiles over them
     std::vector<int32_t> goff(G + 1);
-    HIP_TRY(ctx, hipMemcpyAsync(goff.data(), w.goff, sizeof(int32_t) * (G + 1), hipMemcpyDeviceToHost, s));
+    {
+        PackParts pp{};
+        pp.src[0] = reinterpret_cast<const uint32_t *>(w.goff);
+        pp.words[0] = G + 1;
+        pp.n = 1;
+        RUN(ctx, s, "pack_routing",
+            launch_pack_words(pp, reinterpret_cast<uint32_t *>(L->stage_dev + 2 * rows_bytes), s));
+    }
     HIP_TRY(ctx, hipStreamSynchronize(s));
+    memcpy(goff.data(), L->stage + 2 * rows_bytes, sizeof(int32_t) * (G + 1));
     const int P = goff[G];
     if (P != T * (S + k)) return fail(ctx, GTMOE_ERR_DEVICE, "dispatch placed %d positions, expected %d", P, T * (S + k));
     std::vector<int32_t> pgroup(P);
@@ -1334,13 +1372,13 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
         for (int p = goff[g]; p < goff[g + 1]; ++p) pgroup[p] = g;
         for (int p = goff[g]; p < goff[g + 1]; p += bt) ttr.push_back(make_int4(g, p, std::min(bt, goff[g + 1] - p), 0));
     }
-    HIP_TRY(ctx, hipMemcpyAsync(tw.pgroup, pgroup.data(), sizeof(int32_t) * P, hipMemcpyHostToDevice, s));
-    HIP_TRY(ctx, hipMemcpyAsync(tw.tiles_tr, ttr.data(), sizeof(int4) * ttr.size(), hipMemcpyHostToDevice, s));
+    tw.pgroup = tables.put(pgroup);
+    tw.tiles_tr = tables.put(ttr);
+    put_outer_tiles(tables, goff, tw.ot);
+    HIP_TRY(ctx, tables.send(s));
     tw.P = P;
     tw.ntiles_tr = (int)ttr.size();
     tw.tile_tr = bt;
-    rc = upload_outer_tiles(ctx, goff, tw.ot, s);
-    if (rc != GTMOE_OK) return rc;
 
     // the bare products x W^T by the decode GEMV kernels (raw mode, over the
     // dispatch's slices), then the adapter terms and the biases
@@ -1402,11 +1440,13 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
     RUN(ctx, s, "lora_down", launch_lora_down(ld, w.hidden32, hp, nullptr, tw.u_down, s));
     RUN(ctx, s, "lora_up_bias", launch_lora_up_bias(ld, tw.u_down, w.slot_out, d, L->down.biases, s));
     RUN(ctx, s, "combine",
-        launch_combine(T, d, S, k, w.slot_out, false, w.pos, w.gates32, nullptr, nullptr, w.y64, s));
-    HIP_TRY(ctx, hipMemcpyAsync(outputs, w.y64, sizeof(double) * T * d, hipMemcpyDeviceToHost, s));
-    L->last_load.assign(E, 0);
-    HIP_TRY(ctx, hipMemcpyAsync(L->last_load.data(), w.load, sizeof(int32_t) * E, hipMemcpyDeviceToHost, s));
+        launch_combine(T, d, S, k, w.slot_out, false, w.pos, w.gates32, nullptr,
+                       reinterpret_cast<float *>(L->stage_dev + rows_bytes), nullptr, s));
+    L->last_load.resize(E);
+    for (int e = 0; e < E; ++e) L->last_load[e] = goff[S + e + 1] - goff[S + e];
     HIP_TRY(ctx, hipStreamSynchronize(s));
+    const float *hy = reinterpret_cast<const float *>(L->stage + rows_bytes);
+    for (size_t i = 0; i < nvals; ++i) outputs[i] = (double)hy[i];
     mark_forward(L, T, GTMOE_PATH_FP32, s);
     L->load_on_host = true;
     L->relaunch_ready = false;
@@ -1425,6 +1465,8 @@ int32_t adapter_backward(gtmoe_layer *L, int T, const double *output_grads, doub
     hipStream_t s = ctx->stream;
     const int d = L->d, dp = L->dp, hp = L->hp, E = L->E, S = L->S, k = L->k, P = tw.P;
     const float limit = (float)L->desc.clamp_limit;
+    const int32_t rc = ensure_stage(L, sizeof(double) * T * d);
+    if (rc != GTMOE_OK) return rc;
     HIP_TRY(ctx, hipMemcpyAsync(tw.og, output_grads, sizeof(double) * T * d, hipMemcpyHostToDevice, s));
     // down layer: its pre-activation gradient is the expert output gradient
     RUN(ctx, s, "expert_output_grad",
@@ -1466,8 +1508,9 @@ int32_t adapter_backward(gtmoe_layer *L, int T, const double *output_grads, doub
                                  L->ad_router.dB, tw.outer, s));
         RUN(ctx, s, "add_rows", launch_add_rows_f64(tw.dxr, dp, d, T, tw.dx, s));
     }
-    HIP_TRY(ctx, hipMemcpyAsync(input_grads, tw.dx, sizeof(double) * T * d, hipMemcpyDeviceToHost, s));
+    HIP_TRY(ctx, hipMemcpyAsync(L->stage, tw.dx, sizeof(double) * T * d, hipMemcpyDeviceToHost, s));
     HIP_TRY(ctx, hipStreamSynchronize(s));
+    memcpy(input_grads, L->stage, sizeof(double) * T * d);
     return GTMOE_OK;
 }
 
@@ -2736,17 +2779,33 @@ int32_t gtmoe_layer_adapter_gradients(gtmoe_layer *L, int32_t role, int32_t inde
     int g = 0;
     AdapterSet *a = adapter_of(L, role, index, &g);
     if (!a) return L->has_adapters ? GTMOE_ERR_INVALID_ARGUMENT : GTMOE_ERR_NOT_READY;
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    if (down_grad) {
-        std::vector<double> A((size_t)a->R * a->kin);
-        HIP_TRY(ctx, hipMemcpy(A.data(), a->dA + (size_t)g * a->R * a->kin, A.size() * sizeof(double),
-                               hipMemcpyDeviceToHost));
-        for (int j = 0; j < a->R; ++j)
-            for (int i = 0; i < a->width; ++i) down_grad[(size_t)j * a->width + i] = A[(size_t)j * a->kin + i];
+    // both arrays into the layer's pinned staging by one kernel on the stream,
+    // one wait, then to the caller (two blocking copies to pageable memory and
+    // a repacking took 31.7 us a call, 25.0 so: 16 ranks of a 1024 x 512
+    // matrix)
+    const size_t an = down_grad ? (size_t)a->R * a->kin : 0, bn = up_grad ? (size_t)a->rows * a->R : 0;
+    if (an + bn == 0) return GTMOE_OK;
+    const size_t boff = align_up(an * sizeof(double), 64);
+    const int32_t rc = ensure_stage(L, boff + bn * sizeof(double));
+    if (rc != GTMOE_OK) return rc;
+    PackParts pp{};
+    if (an) {
+        pp.src[pp.n] = reinterpret_cast<const uint32_t *>(a->dA + (size_t)g * an);
+        pp.words[pp.n++] = (int)(2 * an);
     }
-    if (up_grad)
-        HIP_TRY(ctx, hipMemcpy(up_grad, a->dB + (size_t)g * a->rows * a->R, (size_t)a->rows * a->R * sizeof(double),
-                               hipMemcpyDeviceToHost));
+    if (bn) {
+        pp.src[pp.n] = reinterpret_cast<const uint32_t *>(a->dB + (size_t)g * bn);
+        pp.words[pp.n++] = (int)(2 * bn);
+    }
+    RUN(ctx, ctx->stream, "pack_gradients",
+        launch_pack_words(pp, reinterpret_cast<uint32_t *>(L->stage_dev), ctx->stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    const double *ha = reinterpret_cast<const double *>(L->stage);
+    if (an && a->kin == a->width) memcpy(down_grad, ha, an * sizeof(double));
+    else if (an)
+        for (int j = 0; j < a->R; ++j)
+            memcpy(down_grad + (size_t)j * a->width, ha + (size_t)j * a->kin, sizeof(double) * a->width);
+    if (bn) memcpy(up_grad, L->stage + boff, bn * sizeof(double));
     return GTMOE_OK;
 }
 
