@@ -618,7 +618,7 @@ int32_t prepare_and_route(gtmoe_layer *L, int T, const Inputs &in, const int64_t
             f.pend_k = pend->k;
         }
         // the fp32 path's kernels find their own tokens from the choices
-        L->skipped_dispatch = path == GTMOE_PATH_FP32 && T <= kSelfDispatchMaxTokens;
+        L->skipped_dispatch = path == GTMOE_PATH_FP32 && self_dispatches(T, L->k, L->dp, L->hp);
         // When the batch holds at least one entry per expert, the gate/up
         // kernel that follows streams most groups' rows, shared groups first
         // and then routed experts in order: the routing launch reads the

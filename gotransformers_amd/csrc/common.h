@@ -120,9 +120,18 @@ struct GemvArgs {
 
 // Tokens per work slice of the GEMV path (the dispatch's tile size there).
 constexpr int kGemvSlice = 8;
-// Up to this many tokens the fp32 path's expert kernels find their own
-// tokens in the routing choices and no dispatch launch runs.
-constexpr int kSelfDispatchMaxTokens = 64;
+// Few tokens: the fp32 path's expert kernels find their own tokens in the
+// routing choices and no dispatch launch runs.  Up to 64 tokens always; in
+// layers of at most 512 x 512 values, whose expert kernels are so short that
+// the launch saved outweighs the longer scans, up to 512 choices (d = 256, h =
+// 512, 8 Float32 experts, k = 2: 70 tokens 21.1 -> 18.0 us, 128 23.0 -> 20.5,
+// 256 27.5 -> 25.9; larger layers lose: d = 2048, h = 1024, 64 + 1 FP4
+// experts, k = 4, 113 tokens 96.5 against 98.8).  At most 64 passes of
+// kGemvSlice tokens per expert (T <= 512).
+inline bool self_dispatches(int T, int k, int dp, int hp)
+{
+    return T <= 64 || (T * k <= 512 && dp <= 512 && hp <= 512);
+}
 
 // Launchers of the decode expert kernels (each returns the hipError_t of its launch).
 hipError_t launch_gemv_gateup(const GemvArgs &a, int precision, int max_slices, hipStream_t s);

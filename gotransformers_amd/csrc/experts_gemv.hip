@@ -590,7 +590,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 4) void gemv_kernel(GemvArgs
                 for (int i = e0; i < e1; ++i) {
                     const int m = max(0, (hist[i] - 1) / kGemvSlice);
                     if (j >= before && j < before + m) {
-                        found[1] = i * 64 + (j - before + 1);  // T <= 64: at most 8 passes
+                        found[1] = i * 64 + (j - before + 1);  // T <= 512: at most 64 passes
                     }
                     before += m;
                 }

@@ -585,17 +585,20 @@ def test_stack_routing_outputs_need_one_k(ctx):
 
 
 @pytest.mark.parametrize("prec", [FLOAT32, INT8, FP4])
-@pytest.mark.parametrize("E,k,T", [(1, 1, 9), (4, 2, 8), (4, 2, 17), (64, 4, 64), (200, 3, 33)])
+@pytest.mark.parametrize("E,k,T", [(1, 1, 9), (4, 2, 8), (4, 2, 17), (64, 4, 64), (200, 3, 33), (1, 1, 512),
+                                   (3, 2, 256), (3, 2, 257)])
 def test_crowded_experts_in_few_tokens(ctx, prec, E, k, T):
     """Hash routing with one id on every row but a few: k experts hold nearly
     every token, so the decode kernels' passes of 8 tokens beyond an expert's
     first run in the extra workgroups.  K of 9 and 5 chunks of 64 values split
-    unevenly over four and eight waves."""
+    unevenly over four and eight waves; more than 64 tokens through a layer of
+    at most 512 x 512 values, up to its limit of 512 choices and past it."""
     say(f"crowded experts E={E} k={k} T={T} precision {prec}")
-    spec = make_moe(gt.encode_rows, d=576, h=300, E=E, k=k, S=1, precision=prec, seed=31, std=0.05, bias_std=0.02,
+    d = 576 if T <= 64 else 200
+    spec = make_moe(gt.encode_rows, d=d, h=300, E=E, k=k, S=1, precision=prec, seed=31, std=0.05, bias_std=0.02,
                     use_hash=True)
     rng = np.random.default_rng(T)
-    x = rng.normal(size=(T, 576))
+    x = rng.normal(size=(T, d))
     ids = np.full(T, 7, np.int64)
     ids[::5] = rng.integers(0, 1000, size=len(ids[::5]))
     m = gt.MixtureOfExperts.from_spec(ctx, spec)
