@@ -1658,6 +1658,143 @@ __global__ __launch_bounds__(1024) void route_token_kernel(FusedArgs a)
     topk_token<EPL>(lg, t, a.E, a.k, bal, lane, a.chosen, a.gates, a.gates32, TopkScratch{lg, cand, stk});
 }
 
+// Two tokens per workgroup, for batches of more tokens than the GPU holds
+// routing workgroups (1024 threads at up to 128 registers: one per CU, so 257
+// tokens took two rounds): route_token_kernel's arithmetic, fp32 rows, no
+// pending combine, widths that are multiples of 4 up to 2048.  Every wave
+// keeps both rows in registers and reads each router row once for both; waves
+// 0 and 1 run the two top-ks.  d = 2048, 64 experts, k = 4, 333 tokens 19.8 ->
+// 12.7 us.
+template <bool NORM, int EPL, int NX>
+__global__ __launch_bounds__(1024) void route_pair_kernel(FusedArgs a)
+{
+    __shared__ double lg[2][kMaxExperts];
+    __shared__ int cand[2][kMaxExperts];
+    __shared__ int stk[2][3 * kSortStack];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t0 = 2 * blockIdx.x;
+    const bool second = t0 + 1 < a.T;  // the last workgroup may hold one token, which it then repeats
+    const float *rows[2] = {reinterpret_cast<const float *>(a.x) + (size_t)t0 * a.d,
+                            reinterpret_cast<const float *>(a.x) + (size_t)(second ? t0 + 1 : t0) * a.d};
+    double bias_l = 0.0;  // router bias of expert wave + 16 j in lane j
+    double bal[EPL];      // balance biases (waves 0 and 1)
+    if (wave + 16 * lane < a.E) bias_l = a.bias[wave + 16 * lane];
+    if (wave < 2) load_balance<EPL>(a.balance, a.E, lane, bal);
+    static_assert(NX <= 8, "run j of token u is written by wave 8 u + j");
+    const int run = 4 * lane + 256 * (wave & 7);
+    float4 nv = make_float4(1.f, 1.f, 1.f, 1.f);
+    if (NORM && (wave & 7) < NX && run < a.d) nv = *reinterpret_cast<const float4 *>(a.norm + run);
+    float4 xv[2][NX];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < NX; ++j) xv[u][j] = in4(rows[u], min(4 * lane + 256 * j, a.d - 4));
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < NX; ++j)
+            if (4 * lane + 256 * j >= a.d) xv[u][j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    float inv[2] = {1.0f, 1.0f};
+    if (NORM) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < NX; ++j) {
+                ss = fmaf(xv[u][j].x, xv[u][j].x, ss);
+                ss = fmaf(xv[u][j].y, xv[u][j].y, ss);
+                ss = fmaf(xv[u][j].z, xv[u][j].z, ss);
+                ss = fmaf(xv[u][j].w, xv[u][j].w, ss);
+            }
+            ss = wave_sum(ss);
+            inv[u] = 1.0f / sqrtf(ss / (float)a.d + 1e-6f);
+        }
+    }
+    // prepared rows
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < NX; ++j) {
+            const int i = 4 * lane + 256 * j, t = t0 + u;
+            if (8 * u + j == wave && i < a.kp && t < a.T) {  // i < d, or padding (xv holds zeros there)
+                float4 v = xv[u][j];
+                if (NORM) {
+                    v.x = v.x * inv[u] * nv.x;
+                    v.y = v.y * inv[u] * nv.y;
+                    v.z = v.z * inv[u] * nv.z;
+                    v.w = v.w * inv[u] * nv.w;
+                    if (i >= a.d) v = make_float4(0.f, 0.f, 0.f, 0.f);
+                }
+                if (a.xf) *reinterpret_cast<float4 *>(a.xf + (size_t)t * a.kp + i) = v;
+                if (a.xb) {
+                    const uint2 b = make_uint2((uint32_t)bf16_bits(v.x) | ((uint32_t)bf16_bits(v.y) << 16),
+                                               (uint32_t)bf16_bits(v.z) | ((uint32_t)bf16_bits(v.w) << 16));
+                    *reinterpret_cast<uint2 *>(a.xb + (size_t)t * a.kp + i) = b;
+                }
+            }
+        }
+    if (a.zero_out)
+        for (int i = threadIdx.x; i < (second ? 2 : 1) * a.d; i += 1024) a.zero_out[(size_t)t0 * a.d + i] = 0.f;
+    // router rows in flight per wave: both rows of a pair of experts up to d =
+    // 1024, one above (the tokens' rows hold 64 registers there)
+    constexpr int ROWS = NX <= 4 ? 2 : 1;
+    for (int e0 = wave; e0 < a.E; e0 += 16 * ROWS) {
+        float4 p[ROWS][NX];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            const float *w = a.w + (size_t)(e0 + 16 * r < a.E ? e0 + 16 * r : e0) * a.kp;
+#pragma unroll
+            for (int j = 0; j < NX; ++j) p[r][j] = *reinterpret_cast<const float4 *>(w + min(4 * lane + 256 * j, a.kp - 4));
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            float dot[2] = {0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < NX; ++j)
+                if (4 * lane + 256 * j < a.kp) {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        dot[u] = fmaf(xv[u][j].x, p[r][j].x, dot[u]);
+                        dot[u] = fmaf(xv[u][j].y, p[r][j].y, dot[u]);
+                        dot[u] = fmaf(xv[u][j].z, p[r][j].z, dot[u]);
+                        dot[u] = fmaf(xv[u][j].w, p[r][j].w, dot[u]);
+                    }
+                }
+            const int e = e0 + 16 * r;
+            const double b = lane_double(bias_l, min(e, a.E - 1) / 16);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const float v = wave_sum(dot[u]);
+                if (lane == 0 && e < a.E) lg[u][e] = (double)(v * inv[u]) + b;
+            }
+        }
+    }
+    __syncthreads();
+    if (wave >= (second ? 2 : 1)) return;
+    topk_token<EPL>(lg[wave], t0 + wave, a.E, a.k, bal, lane, a.chosen, a.gates, a.gates32,
+                    TopkScratch{lg[wave], cand[wave], stk[wave]});
+}
+
+constexpr int kPairTokens = 256;  // more tokens: two per workgroup
+
+template <bool NORM, int NX>
+static hipError_t launch_pair_nx(const FusedArgs &a, hipStream_t s)
+{
+    const dim3 grid((a.T + 1) / 2);
+    if (a.E <= 64) hipLaunchKernelGGL((route_pair_kernel<NORM, 1, NX>), grid, dim3(1024), 0, s, a);
+    else if (a.E <= 128) hipLaunchKernelGGL((route_pair_kernel<NORM, 2, NX>), grid, dim3(1024), 0, s, a);
+    else hipLaunchKernelGGL((route_pair_kernel<NORM, 4, NX>), grid, dim3(1024), 0, s, a);
+    return hipGetLastError();
+}
+
+template <bool NORM>
+static hipError_t launch_pair(const FusedArgs &a, hipStream_t s)
+{
+    if (a.kp <= 256) return launch_pair_nx<NORM, 1>(a, s);
+    if (a.kp <= 1024) return launch_pair_nx<NORM, 4>(a, s);
+    return launch_pair_nx<NORM, 8>(a, s);
+}
+
 bool fused_route_fits(int T, int k, int kp) { return T >= 1 && T * k <= kFusedMaxTK && T <= 1024 && kp <= 4096; }
 
 // Parts per token: up to 128 workgroups in all, at least 32 experts per
@@ -1703,6 +1840,8 @@ hipError_t launch_route_fused(const FusedArgs &a, bool input_f64, bool hash, boo
         return hipErrorInvalidValue;
     hipError_t e;
     if (input_f64) e = a.norm ? launch_token_typed<double, true>(a, hash, s) : launch_token_typed<double, false>(a, hash, s);
+    else if (a.T > kPairTokens && !hash && a.parts == 1 && !a.pend_slot && a.d % 4 == 0 && a.kp <= 2048)
+        e = a.norm ? launch_pair<true>(a, s) : launch_pair<false>(a, s);
     else e = a.norm ? launch_token_typed<float, true>(a, hash, s) : launch_token_typed<float, false>(a, hash, s);
     if (e != hipSuccess || !dispatch) return e;
     hipLaunchKernelGGL(dispatch_kernel, dim3(1), dim3(1024), 0, s, a.chosen, a.T, a.k, a.E, a.S, a.bm, a.load,

@@ -663,3 +663,31 @@ def test_scores_that_share_their_upper_bits(ctx, E, k):
         want = oracle.route_from_logits(logits, k, b)
         assert np.array_equal(got.chosen, want.chosen)
         assert np.array_equal(got.gates.view(np.int64), want.gates.view(np.int64))
+
+
+@pytest.mark.parametrize("d,E,k", [(64, 5, 2), (260, 128, 7), (1024, 16, 2), (1500, 200, 3), (2048, 64, 4)])
+@pytest.mark.parametrize("T", [257, 258])
+def test_two_tokens_per_routing_workgroup(ctx, d, E, k, T):
+    """More than 256 tokens route two per workgroup: choices, gates and
+    outputs to the bit as in two calls of one token per workgroup, plain and
+    behind an RMSNorm (the last workgroup holds one or two tokens)."""
+    say(f"paired routing d={d} E={E} k={k} T={T}")
+    spec = make_moe(gt.encode_rows, d=d, h=16, E=E, k=k, S=1, precision=INT8, seed=61, std=0.05)
+    rng = np.random.default_rng(62)
+    x = rng.normal(size=(T, d))
+    m = gt.MixtureOfExperts.from_spec(ctx, spec)
+    try:
+        m.set_norm_weights(rng.uniform(0.5, 1.5, d))
+        y = m.forward(x, path=gt.PATH_BF16)
+        r = m.last_routing()
+        s = gt.stack_forward([m], x, path=gt.PATH_BF16, with_routing=True)
+        parts = []
+        for rows in (x[:129], x[129:]):
+            yp = m.forward(rows, path=gt.PATH_BF16)
+            rp = m.last_routing()
+            parts.append((yp, rp.chosen, rp.gates, *gt.stack_forward([m], rows, path=gt.PATH_BF16, with_routing=True)))
+    finally:
+        m.destroy()
+    yp, cp, gp, sx, sc, sg = (np.concatenate(v, axis=1 if v[0].ndim == 3 else 0) for v in zip(*parts))
+    assert np.array_equal(r.chosen, cp) and np.array_equal(r.gates, gp) and np.array_equal(y, yp)
+    assert np.array_equal(s[1], sc) and np.array_equal(s[2], sg) and np.array_equal(s[0], sx)
