@@ -49,7 +49,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int BN = 256;    // weight rows per tile (gate/up: 128 neurons x 2)
+constexpr int BN = 256;    // weight rows per tile (gate/up: 128 neurons x 2; down over few tiles: 128)
 constexpr int BK = 64;     // K per pipeline step (4 scale blocks)
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -228,11 +228,12 @@ __device__ __forceinline__ char *pick(char *b0, char *b1, char *b2)
 
 }  // namespace
 
-// One tile whose positions lie in its first MI 32-row blocks (M <= 32 MI):
+// One tile whose positions lie in its first MI 32-row blocks (M <= 32 MI),
+// NJ column tiles of 32 per wave (gate/up: 2; down: 2 or 1):
 // the blocks past them are neither loaded nor multiplied.  b0, b1, b2: the
 // three activation buffers (buf_bytes of LDS each, separate arrays, so that
 // the compiler tells their accesses apart).
-template <int PREC, bool GATEUP, int MI, int BM>
+template <int PREC, bool GATEUP, int MI, int BM, int NJ>
 __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1, char *b2, int g, int p0, int M,
                                           int ntile)
 {
@@ -277,11 +278,11 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
     // weights: the wave's two column tiles (gate/up: the same 32 neurons of
     // gate and up; down: 64 consecutive rows), a group's matrices as buffer
     // resources; columns past n read zeros and are not written
-    GroupSrc bsrc[2];
-    uint32_t bvo[2], bvs[2];
+    GroupSrc bsrc[NJ];
+    uint32_t bvo[NJ], bvs[NJ];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int n = GATEUP ? ntile * (BN / 2) + wave * 32 + col : ntile * BN + wave * 64 + j * 32 + col;
+    for (int j = 0; j < NJ; ++j) {
+        const int n = GATEUP ? ntile * (BN / 2) + wave * 32 + col : ntile * (128 * NJ) + wave * (32 * NJ) + j * 32 + col;
         const void *w = GATEUP ? (j ? a.w1 : a.w0) : a.w0;
         const float *sc = GATEUP ? (j ? a.s1 : a.s0) : a.s0;
         bsrc[j].codes = __builtin_amdgcn_make_buffer_rsrc(
@@ -307,11 +308,11 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
     // neurons' biases: the epilogue has nothing to load.  The biases are
     // requested here and copied in after the prologue, whose counted waits
     // cover them (they are the oldest loads).
-    int nbase[2];
-    floatx16 binit[2], acc[MI][2];
+    int nbase[NJ];
+    floatx16 binit[NJ], acc[MI][NJ];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        nbase[j] = GATEUP ? ntile * (BN / 2) + wave * 32 : ntile * BN + wave * 64 + j * 32;
+    for (int j = 0; j < NJ; ++j) {
+        nbase[j] = GATEUP ? ntile * (BN / 2) + wave * 32 : ntile * (128 * NJ) + wave * (32 * NJ) + j * 32;
         const float *bias = (GATEUP && j ? a.b1 : a.b0) + (size_t)g * a.n;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -351,8 +352,8 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
     const int nsteps = a.kp / BK;
     constexpr int NS = PREC == kFloat32 ? 2 : 3;
     constexpr int UNROLL = NS == 3 ? 3 : 6;
-    BRaw<PREC> bq[NS][2];  // [stage][column tile]
-    constexpr int NB = PREC == kInt8 ? 6 : PREC == kFP4 ? 4 : 8;
+    BRaw<PREC> bq[NS][NJ];  // [stage][column tile]
+    constexpr int NB = NJ * (PREC == kInt8 ? 3 : PREC == kFP4 ? 2 : 4);
     constexpr int VM = 2 * NB + MI;
     static_assert(VM < 64, "vmcnt holds six bits");
     // s_waitcnt vmcnt(n) lgkmcnt(0), expcnt not waited for
@@ -369,11 +370,11 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
                 asrc, (__attribute__((address_space(3))) void *)(buf + (32 * i + 8 * wave) * 128), 16, aoff[i],
                 k0 * 2, 0, 0);
     };
-    auto load_b = [&](BRaw<PREC> (&q)[2], int step) {
+    auto load_b = [&](BRaw<PREC> (&q)[NJ], int step) {
         const int m = min(step, nsteps - 1);
         // pair p of the step: this lane's block is 2p + h (FP4: 2h + p)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NJ; ++j) {
 #pragma unroll
             for (int p = 0; p < 2; ++p) load_block<PREC>(q[j], p, bsrc[j], bvo[j], m, p);
             load_scales<PREC>(q[j], bsrc[j], bvs[j], m);
@@ -391,13 +392,13 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
     // work hides under the matrix cores: the scheduling groups below ask for
     // one MFMA, then a share of the VALU instructions (four with all four
     // row blocks), in turn.
-    auto dequant_pair = [&](const BRaw<PREC> (&q)[2], int p, bf16x8 (&out)[2][2]) {
+    auto dequant_pair = [&](const BRaw<PREC> (&q)[NJ], int p, bf16x8 (&out)[NJ][2]) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int s2 = 0; s2 < 2; ++s2) out[j][s2] = dequant_half<PREC>(q[j], p, s2);
     };
-    auto mfma_pair = [&](const char *buf, int p, const bf16x8 (&bfp)[2][2]) {
+    auto mfma_pair = [&](const char *buf, int p, const bf16x8 (&bfp)[NJ][2]) {
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
             // k-values of this MFMA step: lanes of half h carry values
@@ -411,7 +412,7 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < NJ; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfp[j][s2], af[i], acc[i][j], 0, 0, 0);
         }
     };
@@ -420,13 +421,13 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
         for (int s2 = 0; s2 < 2; ++s2) {
             __builtin_amdgcn_sched_group_barrier(0x100, MI, 0);  // the LDS reads of the A operands
 #pragma unroll
-            for (int m = 0; m < 2 * MI; ++m) {
+            for (int m = 0; m < NJ * MI; ++m) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                   // one MFMA
                 __builtin_amdgcn_sched_group_barrier(0x002, (16 + MI - 1) / MI, 0);  // VALU
             }
         }
     };
-    bf16x8 bfa[2][2], bfb[2][2];  // B operands of the current and the next half step
+    bf16x8 bfa[NJ][2], bfb[NJ][2];  // B operands of the current and the next half step
     // step k of the pipeline (U = k % UNROLL); bfa holds pair 0 of step k.
     // The last steps, after the loop, wait for all their loads instead: the
     // compiler drops their weight loads (nothing reads them), which leaves
@@ -475,7 +476,7 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = binit[j];
+        for (int j = 0; j < NJ; ++j) acc[i][j] = binit[j];
     int k = 0;
     for (; k + UNROLL <= nsteps; k += UNROLL) {
         step(std::integral_constant<int, 0>{}, k, loop_wait);
@@ -543,7 +544,7 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
         store_tile<BM>(a, n8 <= a.ldo ? n8 : a.n, os0, os1, p0, M, [&](int c) { return ntile * (BN / 2) + c; });
     } else {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NJ; ++j) {
             // one column tile of every wave per pass: tile column c is output
             // column ntile * 256 + (c / 32) * 64 + j * 32 + c % 32
 #pragma unroll
@@ -554,14 +555,14 @@ __device__ __forceinline__ void gemm_tile(const MfmaArgs &a, char *b0, char *b1,
                     put4(i, q, pack_bf16(acc[i][j][r], acc[i][j][r + 1]), pack_bf16(acc[i][j][r + 2], acc[i][j][r + 3]));
                 }
             __syncthreads();
-            store_tile<BM>(a, a.n, os0, os1, p0, M, [&](int c) { return ntile * BN + (c >> 5) * 64 + j * 32 + (c & 31); });
-            if (j == 0) __syncthreads();  // the next pass rewrites the LDS tile
+            store_tile<BM>(a, a.n, os0, os1, p0, M, [&](int c) { return ntile * (128 * NJ) + (c >> 5) * (32 * NJ) + j * 32 + (c & 31); });
+            if (j + 1 < NJ) __syncthreads();  // the next pass rewrites the LDS tile
         }
     }
 }
 
-template <int PREC, bool GATEUP, int BM>
-__global__ __launch_bounds__(256, BM == 64 && PREC == kFP4 ? 3 : 2) void mfma_gemm_kernel(MfmaArgs a)
+template <int PREC, bool GATEUP, int BM, int NJ>
+__global__ __launch_bounds__(256, NJ == 1 ? (BM == 64 ? 4 : 3) : BM == 64 && PREC == kFP4 ? 3 : 2) void mfma_gemm_kernel(MfmaArgs a)
 {
     __shared__ __attribute__((aligned(16))) char buf0[buf_bytes<BM>()];
     __shared__ __attribute__((aligned(16))) char buf1[buf_bytes<BM>()];
@@ -582,12 +583,12 @@ __global__ __launch_bounds__(256, BM == 64 && PREC == kFP4 ? 3 : 2) void mfma_ge
     // run as two: the dequantization, the same for any M, then bounds the time
     // anyway)
     if constexpr (BM == 64) {
-        if (M > 32) gemm_tile<PREC, GATEUP, 2, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
-        else gemm_tile<PREC, GATEUP, 1, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
+        if (M > 32) gemm_tile<PREC, GATEUP, 2, BM, NJ>(a, buf0, buf1, buf2, g, p0, M, ntile);
+        else gemm_tile<PREC, GATEUP, 1, BM, NJ>(a, buf0, buf1, buf2, g, p0, M, ntile);
     } else {
-        if (M > 96) gemm_tile<PREC, GATEUP, 4, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
-        else if (M > 64) gemm_tile<PREC, GATEUP, 3, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
-        else gemm_tile<PREC, GATEUP, 2, BM>(a, buf0, buf1, buf2, g, p0, M, ntile);
+        if (M > 96) gemm_tile<PREC, GATEUP, 4, BM, NJ>(a, buf0, buf1, buf2, g, p0, M, ntile);
+        else if (M > 64) gemm_tile<PREC, GATEUP, 3, BM, NJ>(a, buf0, buf1, buf2, g, p0, M, ntile);
+        else gemm_tile<PREC, GATEUP, 2, BM, NJ>(a, buf0, buf1, buf2, g, p0, M, ntile);
     }
 }
 
@@ -643,20 +644,35 @@ hipError_t launch_mfma(const MfmaArgs &a, int precision, int max_tiles, hipStrea
     if (a.a_rows <= 0 || a.a_rows * a.lda * 2 > 0x7fffffffLL || a.w_group_stride > 0x7fffffffLL ||
         a.s_group_stride * 4 > 0x7fffffffLL)
         return hipErrorInvalidValue;
-    constexpr int COLS = GATEUP ? BN / 2 : BN;  // output columns per tile
     MfmaArgs b = a;
-    b.ntiles_n = (a.n + COLS - 1) / COLS;
-    const dim3 grid((unsigned)((max_tiles + 7) / 8 * 8 * b.ntiles_n));
-    auto launch = [&](auto prec_tag) {
-        constexpr int P = decltype(prec_tag)::value;
-        if (a.bm == 64) hipLaunchKernelGGL((mfma_gemm_kernel<P, GATEUP, 64>), grid, dim3(256), 0, s, b);
-        else hipLaunchKernelGGL((mfma_gemm_kernel<P, GATEUP, 128>), grid, dim3(256), 0, s, b);
+    auto launch = [&](auto prec_tag, auto nj_tag) {
+        constexpr int P = decltype(prec_tag)::value, NJ = decltype(nj_tag)::value;
+        constexpr int COLS = GATEUP ? BN / 2 : 128 * NJ;  // output columns per tile
+        b.ntiles_n = (a.n + COLS - 1) / COLS;
+        const dim3 grid((unsigned)((max_tiles + 7) / 8 * 8 * b.ntiles_n));
+        if (a.bm == 64) hipLaunchKernelGGL((mfma_gemm_kernel<P, GATEUP, 64, NJ>), grid, dim3(256), 0, s, b);
+        else hipLaunchKernelGGL((mfma_gemm_kernel<P, GATEUP, 128, NJ>), grid, dim3(256), 0, s, b);
+    };
+    // Down over few tiles: 128 columns per tile, one column tile per wave, so
+    // that the grid reaches more CUs and its smaller registers three or four
+    // workgroups on each.  Where 256-column tiles (a bound on them) would not
+    // fill the 256 CUs once, twice with 64-position tiles: a layer of d = 1024,
+    // h = 2048, 16 Int8 experts, k = 2 over 128 tokens 57.5 -> 50.8 us, over 800
+    // 81.0 -> 67.9; d = 1000, h = 1201, 14 + 2 Int8, k = 3 over 150 52.2 -> 46.1;
+    // d = 1024, h = 512, 64 + 1 FP4, k = 6 over 150 (268 tiles of 64 positions)
+    // 48.0 -> 46.2, but over 600 (128 positions) 73.2 against 75.6.
+    auto launch_nj = [&](auto prec_tag) {
+        if constexpr (!GATEUP) {
+            if ((long long)max_tiles * ((a.n + BN - 1) / BN) < (a.bm == 64 ? 512 : 256))
+                return launch(prec_tag, std::integral_constant<int, 1>{});
+        }
+        launch(prec_tag, std::integral_constant<int, 2>{});
     };
     if (a.bm != 64 && a.bm != 128) return hipErrorInvalidValue;
     switch (precision) {
-    case kInt8: launch(std::integral_constant<int, kInt8>{}); break;
-    case kFP4: launch(std::integral_constant<int, kFP4>{}); break;
-    case kFloat32: launch(std::integral_constant<int, kFloat32>{}); break;
+    case kInt8: launch_nj(std::integral_constant<int, kInt8>{}); break;
+    case kFP4: launch_nj(std::integral_constant<int, kFP4>{}); break;
+    case kFloat32: launch_nj(std::integral_constant<int, kFloat32>{}); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

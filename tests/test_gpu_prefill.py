@@ -347,3 +347,23 @@ def test_tiles_of_64_and_128_positions(ctx, prec, T):
         ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates)
         e = rel_err(y, ref.outputs)
         assert e <= BF16_TOL, e
+
+
+@pytest.mark.parametrize("prec", [FLOAT32, INT8, FP4])
+@pytest.mark.parametrize("d", [1800, 1000])
+def test_down_with_128_and_256_columns_per_tile(ctx, prec, d):
+    """64 experts and 200 tokens give 81 tiles of 64 positions at most: eight
+    256-column tiles of d = 1800 run as they are, four of d = 1000 are split in
+    two."""
+    say(f"down column tiles d={d} precision {prec}")
+    spec = make_moe(gt.encode_rows, d=d, h=64, E=64, k=4, S=1, precision=prec, seed=71, std=0.05, bias_std=0.02)
+    x = np.random.default_rng(72).normal(size=(200, d))
+    m = gt.MixtureOfExperts.from_spec(ctx, spec)
+    try:
+        y = m.forward(x, path=gt.PATH_BF16)
+        r = m.last_routing()
+    finally:
+        m.destroy()
+    ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates, threads=16)
+    e = rel_err(y, ref.outputs)
+    assert e <= BF16_TOL, e
