@@ -553,6 +553,13 @@ struct PendingCombine {
     int S, k, d;
 };
 
+// Whether T tokens of this layer take the fused routing launch; pending: it
+// would also have to do the previous stack layer's combine.
+bool routes_fused(const gtmoe_layer *L, int T, bool f64, bool pending)
+{
+    return fused_route_fits(T, L->k, L->dp, !f64 && !pending && !L->desc.use_hash_routing && L->d % 4 == 0);
+}
+
 // Input preparation, routing and dispatch.  Few tokens: one fused launch.
 // Otherwise: convert or RMSNorm into ws.xf / ws.xb, router and top-k (or hash
 // routing), then the dispatch.  token_ids: device pointer (hash routing).
@@ -576,7 +583,7 @@ int32_t prepare_and_route(gtmoe_layer *L, int T, const Inputs &in, const int64_t
     // the dispatch's per-group tile prefix counts MFMA m-tiles on the bf16
     // path and token slices on the fp32 path
     const int bm = path == GTMOE_PATH_BF16 ? mfma_tile_m(T, L->k, L->E) : kGemvSlice;
-    if (fused_route_fits(T, L->k, L->dp)) {
+    if (routes_fused(L, T, in.f64, pend != nullptr)) {
         FusedArgs f{};
         f.x = in.x;
         f.norm = in.norm ? L->norm_w : nullptr;
@@ -2233,11 +2240,11 @@ static int32_t stack_run(gtmoe_layer *const *layers, int32_t n_layers, int32_t T
         gtmoe_layer *N = l + 1 < n_layers ? layers[l + 1] : nullptr;
         // on the fp32 path the next layer's routing kernel, which reads x
         // anyway, does this layer's combine (one launch fewer per layer)
-        if (N && path == GTMOE_PATH_FP32 && fused_route_fits(T, N->k, N->dp)) {
+        if (N && path == GTMOE_PATH_FP32 && routes_fused(N, T, false, true)) {
             pending = PendingCombine{w.slot_out, pos, w.gates32, L->S, L->k, L->d};
             have_pending = true;
         } else if (N && path == GTMOE_PATH_BF16 && choose_path(N, T, flags) == GTMOE_PATH_BF16 &&
-                   !fused_route_fits(T, N->k, N->dp) && N->d == N->dp && combine_norm_fits(L->d, true)) {
+                   !routes_fused(N, T, false, false) && N->d == N->dp && combine_norm_fits(L->d, true)) {
             // on the bf16 path the combine, which holds whole rows, also does
             // the next layer's RMSNorm: its bf16 rows and inverse RMS
             rc = ensure_workspace(N, T);

@@ -1238,6 +1238,9 @@ hipError_t launch_dispatch(const int32_t *chosen, int T, int k, int E, int S, in
 // raw row, logit = inv_rms * dot(x, wn) + bias.
 // ---------------------------------------------------------------------------
 constexpr int kFusedMaxTK = 2048;  // T*k handled by the two-launch routing
+constexpr int kPairTokens = 256;   // more tokens: two per workgroup, where route_pair_kernel takes them
+constexpr int kPairMaxTK = 4096;   // T*k it is launched for
+constexpr int kPairMaxK = 2048;    // padded row width it holds
 
 __device__ __forceinline__ uint16_t bf16_bits(float f)
 {
@@ -1775,8 +1778,6 @@ __global__ __launch_bounds__(1024) void route_pair_kernel(FusedArgs a)
                     TopkScratch{lg[wave], cand[wave], stk[wave]});
 }
 
-constexpr int kPairTokens = 256;  // more tokens: two per workgroup
-
 template <bool NORM, int NX>
 static hipError_t launch_pair_nx(const FusedArgs &a, hipStream_t s)
 {
@@ -1795,7 +1796,19 @@ static hipError_t launch_pair(const FusedArgs &a, hipStream_t s)
     return launch_pair_nx<NORM, 8>(a, s);
 }
 
-bool fused_route_fits(int T, int k, int kp) { return T >= 1 && T * k <= kFusedMaxTK && T <= 1024 && kp <= 4096; }
+// Batches the routing handles in one launch (with the dispatch behind it); pair:
+// fp32 rows of a width that is a multiple of 4, router routing, nothing pending,
+// so that more than 256 tokens go two per workgroup.  Two rounds of those beat
+// the router, top-k and conversion launches up to T k = 4096 (d = 2048, h =
+// 1024, 64 + 1 FP4 experts, k = 4: 513 tokens 128.7 -> 121.8 us, 1000 170.4 ->
+// 164.5; d = 1024, k = 6, 500 tokens 70.0 -> 59.7; d = 1000, 14 + 2 experts, k
+// = 3, 777 87.5 -> 80.6), not beyond (d = 2048, 128 experts, k = 8, 1000 tokens
+// 258 against 270).
+bool fused_route_fits(int T, int k, int kp, bool pair)
+{
+    const int limit = pair && T > kPairTokens && kp <= kPairMaxK ? kPairMaxTK : kFusedMaxTK;
+    return T >= 1 && T * k <= limit && T <= 1024 && kp <= 4096;
+}
 
 // Parts per token: up to 128 workgroups in all, at least 32 experts per
 // part, at most 8 parts; one for hash routing.  Every part repeats the
@@ -1833,14 +1846,15 @@ static hipError_t launch_token_typed(const FusedArgs &a, bool hash, hipStream_t 
 
 hipError_t launch_route_fused(const FusedArgs &a, bool input_f64, bool hash, bool dispatch, hipStream_t s)
 {
-    if (!fused_route_fits(a.T, a.k, a.kp)) return hipErrorInvalidValue;
+    const bool pair = !input_f64 && !hash && !a.pend_slot && a.d % 4 == 0;
+    if (!fused_route_fits(a.T, a.k, a.kp, pair)) return hipErrorInvalidValue;
     // more than one part needs the arrival counts, and a pending combine
     // then must not be written in place
     if (a.parts < 1 || (a.parts > 1 && (hash || !a.part_cnt || (a.pend_slot && (!a.x_out || a.x_out == a.x)))))
         return hipErrorInvalidValue;
     hipError_t e;
     if (input_f64) e = a.norm ? launch_token_typed<double, true>(a, hash, s) : launch_token_typed<double, false>(a, hash, s);
-    else if (a.T > kPairTokens && !hash && a.parts == 1 && !a.pend_slot && a.d % 4 == 0 && a.kp <= 2048)
+    else if (pair && a.T > kPairTokens && a.parts == 1 && a.kp <= kPairMaxK)
         e = a.norm ? launch_pair<true>(a, s) : launch_pair<false>(a, s);
     else e = a.norm ? launch_token_typed<float, true>(a, hash, s) : launch_token_typed<float, false>(a, hash, s);
     if (e != hipSuccess || !dispatch) return e;

@@ -666,11 +666,12 @@ def test_scores_that_share_their_upper_bits(ctx, E, k):
 
 
 @pytest.mark.parametrize("d,E,k", [(64, 5, 2), (260, 128, 7), (1024, 16, 2), (1500, 200, 3), (2048, 64, 4)])
-@pytest.mark.parametrize("T", [257, 258])
+@pytest.mark.parametrize("T", [257, 258, 511])
 def test_two_tokens_per_routing_workgroup(ctx, d, E, k, T):
     """More than 256 tokens route two per workgroup: choices, gates and
     outputs to the bit as in two calls of one token per workgroup, plain and
-    behind an RMSNorm (the last workgroup holds one or two tokens)."""
+    behind an RMSNorm (the last workgroup holds one or two tokens; 511 tokens of
+    k = 7 pass the one-token kernel's limit of 2048 choices)."""
     say(f"paired routing d={d} E={E} k={k} T={T}")
     spec = make_moe(gt.encode_rows, d=d, h=16, E=E, k=k, S=1, precision=INT8, seed=61, std=0.05)
     rng = np.random.default_rng(62)
@@ -682,7 +683,7 @@ def test_two_tokens_per_routing_workgroup(ctx, d, E, k, T):
         r = m.last_routing()
         s = gt.stack_forward([m], x, path=gt.PATH_BF16, with_routing=True)
         parts = []
-        for rows in (x[:129], x[129:]):
+        for rows in np.array_split(x, 2):  # 128 to 256 tokens: one workgroup each
             yp = m.forward(rows, path=gt.PATH_BF16)
             rp = m.last_routing()
             parts.append((yp, rp.chosen, rp.gates, *gt.stack_forward([m], rows, path=gt.PATH_BF16, with_routing=True)))
