@@ -1798,12 +1798,13 @@ static hipError_t launch_pair(const FusedArgs &a, hipStream_t s)
 
 // Batches the routing handles in one launch (with the dispatch behind it); pair:
 // fp32 rows of a width that is a multiple of 4, router routing, nothing pending,
-// so that more than 256 tokens go two per workgroup.  Two rounds of those beat
-// the router, top-k and conversion launches up to T k = 4096 (d = 2048, h =
+// so that more than 256 tokens go two per workgroup.  One or two rounds of those
+// beat the router, top-k and conversion launches up to T k = 4096 (d = 2048, h =
 // 1024, 64 + 1 FP4 experts, k = 4: 513 tokens 128.7 -> 121.8 us, 1000 170.4 ->
 // 164.5; d = 1024, k = 6, 500 tokens 70.0 -> 59.7; d = 1000, 14 + 2 experts, k
-// = 3, 777 87.5 -> 80.6), not beyond (d = 2048, 128 experts, k = 8, 1000 tokens
-// 258 against 270).
+// = 3, 777 87.5 -> 80.6; layer times, one sweep per limit).  Beyond, the layers
+// differ: k = 6, 1000 tokens 88.0 -> 84.0, but d = 2048, 128 experts, k = 8, 600
+// tokens 224-232 -> 237 and 1000 256-258 -> 270 (ranges: two runs of one route).
 bool fused_route_fits(int T, int k, int kp, bool pair)
 {
     const int limit = pair && T > kPairTokens && kp <= kPairMaxK ? kPairMaxTK : kFusedMaxTK;
