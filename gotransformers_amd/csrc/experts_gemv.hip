@@ -213,25 +213,25 @@ __device__ __forceinline__ void load_tokens(TokenRegs<NQ> &r, __amdgpu_buffer_rs
             float4, __builtin_amdgcn_raw_buffer_load_b128(xin, xo[q], ch * (Chunk<PREC>::CB * 64), 0));
 }
 
-// Panel `panel` of group g as buffer resources.
+// Panel `panel` (down: and the next MATS - 1) of group g as buffer resources.
+// Where the last workgroup's second panel lies past an odd number of panels,
+// it takes the last panel again and its rows are not stored: a resource of no
+// bytes would not do, as the range check counts from the scalar offset.
 template <int PREC, bool GATEUP, int MATS>
 __device__ __forceinline__ void panel_src(const GemvArgs &a, int g, int panel, PanelSrc (&src)[MATS])
 {
 #pragma unroll
     for (int m = 0; m < MATS; ++m) {
-        const int pm = GATEUP ? panel : panel + m;
-        const bool in_matrix = pm * 64 < a.rows;  // the last workgroup's sets may lie past the rows
-        const size_t wpanel = (size_t)pm * 64 * a.row_bytes;
-        const int wbytes = in_matrix ? 64 * a.row_bytes : 0;  // past the rows: every load reads zeros
-        const size_t spanel = (size_t)pm * 64 * a.nblocks;
-        const int sbytes = in_matrix ? 64 * a.nblocks * 4 : 0;
+        const int pm = GATEUP ? panel : min(panel + m, (a.rows - 1) / kPanelRows);
+        const size_t wpanel = (size_t)pm * kPanelRows * a.row_bytes;
+        const size_t spanel = (size_t)pm * kPanelRows * a.nblocks;
         src[m].codes = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<char *>(reinterpret_cast<const char *>(GATEUP && m ? a.w1 : a.w0)) + (size_t)g * a.w_group_stride + wpanel,
-            0, wbytes, kRawBufferWord3);
+            0, kPanelRows * a.row_bytes, kRawBufferWord3);
         if constexpr (PREC != kFloat32)
             src[m].scales = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float *>(GATEUP && m ? a.s1 : a.s0) + (size_t)g * a.s_group_stride + spanel, 0, sbytes,
-                kRawBufferWord3);
+                const_cast<float *>(GATEUP && m ? a.s1 : a.s0) + (size_t)g * a.s_group_stride + spanel, 0,
+                kPanelRows * a.nblocks * 4, kRawBufferWord3);
     }
 }
 

@@ -692,3 +692,18 @@ def test_two_tokens_per_routing_workgroup(ctx, d, E, k, T):
     yp, cp, gp, sx, sc, sg = (np.concatenate(v, axis=1 if v[0].ndim == 3 else 0) for v in zip(*parts))
     assert np.array_equal(r.chosen, cp) and np.array_equal(r.gates, gp) and np.array_equal(y, yp)
     assert np.array_equal(s[1], sc) and np.array_equal(s[2], sg) and np.array_equal(s[0], sx)
+
+
+@pytest.mark.parametrize("prec", [FLOAT32, INT8, FP4])
+@pytest.mark.parametrize("T", [60, 100])
+def test_down_over_an_odd_number_of_panels(ctx, prec, T):
+    """d = 960 is 15 panels of 64 rows and 160 experts make the down kernel
+    take two per wave, so the last workgroup's second panel lies past the
+    matrix; few tokens find their own entries, more go through the dispatch."""
+    say(f"odd down panels T={T} precision {prec}")
+    spec = make_moe(gt.encode_rows, d=960, h=64, E=160, k=4, S=1, precision=prec, seed=81, std=0.05, bias_std=0.02)
+    x = np.random.default_rng(82).normal(size=(T, 960))
+    y, r, _ = run_layer(ctx, spec, x, gt.PATH_FP32)
+    ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates)
+    e = rel_err(y, ref.outputs)
+    assert e <= FP32_TOL, e
