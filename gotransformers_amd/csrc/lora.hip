@@ -332,17 +332,19 @@ __global__ __launch_bounds__(256) void sum_chunks_kernel(const float *__restrict
 
 // The adapters' two projections onto the ranks, as fp32 16x16x4 MFMAs over
 // the position tiles of one group (LoraArgs::otiles):
-//   u[p][j] = sum_i in[row(p)][i] * A[g][j][i]                  (TO_RANK = down)
-//   t[p][j] = scale[g] * sum_n grad[p][n] * B[g][n][j]           (TO_RANK = back)
+//   u[p][j] = sum_i in[row(p)][i] * A[g][j][i]                  (BACK = false)
+//   t[p][j] = scale[g] * sum_n grad[p][n] * B[g][n][j]           (BACK = true)
 // A workgroup takes 16 positions of a tile (blockIdx.z) and 16 ranks, its four
 // waves a quarter of the sum each, in steps of 16 values: a lane reads four
 // consecutive values of its position (and of its rank's row of A, or its
-// rank's column of four rows of B), the four k of four MFMAs.  The waves' sums
-// are added in wave order through LDS.  The loads' latency bounds it, so eight
-// steps are in flight.  (One wave per (position, rank), or one workgroup per
-// position, read the adapter's values for every position: 3584 positions, 16
-// ranks, 512 to 1024 values 17.4 and 16.1 us per launch, now 8.4 and
-// 6.4.)
+// rank's column of four rows of B), the four k of four MFMAs, in two chains of
+// two.  Steps and waves are added in 64 bits: one fp32 accumulator over a
+// wave's quarter put 2.8e-7 of relative error on u at 1024 values and 5.7e-7 at
+// 4096; so it is 6.3e-8 to 7.3e-8 from 256 to 4096 (per-lane sums and a tree
+// over 64 lanes: 7.6e-8 to 1.07e-7), in the same time.  Eight steps' loads are
+// in flight.  (One wave per (position, rank), or one workgroup per position,
+// read the adapter's values for every position: 3584 positions, 16 ranks, 512
+// to 1024 values 17.1 and 15.9 us per launch, 8.3 and 6.4 as here.)
 constexpr int kOpPositions = 64;  // positions of a tile at most
 constexpr int kRkPositions = 16;  // positions of a workgroup
 constexpr int kRkStep = 16;       // values per step
@@ -352,7 +354,7 @@ template <bool BACK>
 __global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const float *__restrict__ in, int ld_in,
                                                            const int32_t *__restrict__ in_tok, float *__restrict__ out)
 {
-    __shared__ float red[4][4][64];
+    __shared__ double red[4][4][64];
     const int4 td = a.otiles[blockIdx.x];
     const int g = td.x, p0 = td.y + kRkPositions * blockIdx.z, m = td.z - kRkPositions * (int)blockIdx.z;
     if (m <= 0) return;  // workgroup-uniform
@@ -367,7 +369,7 @@ __global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const flo
     const float *ad = BACK ? a.B + (size_t)g * a.rows * a.R + jc : a.A + ((size_t)g * a.R + jc) * a.kin;
     const int steps = (nval + kRkStep - 1) / kRkStep;
     const int s0 = wave * steps / 4, s1 = (wave + 1) * steps / 4;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int sb = s0; sb < s1; sb += kRkDepth) {
         f32x4 x[kRkDepth], w[kRkDepth];
 #pragma unroll
@@ -393,9 +395,14 @@ __global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const flo
         }
 #pragma unroll
         for (int q = 0; q < kRkDepth; ++q) {
-            if (sb + q >= s1) break;  // wave-uniform
+            f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q][e], w[q][e], acc, 0, 0, 0);
+            for (int e = 0; e < 4; e += 2) {
+                a = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q][e], w[q][e], a, 0, 0, 0);
+                b = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q][e + 1], w[q][e + 1], b, 0, 0, 0);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[v] += sb + q < s1 ? (double)(a[v] + b[v]) : 0.0;
         }
     }
 #pragma unroll
@@ -405,7 +412,7 @@ __global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const flo
     // finishes register w
     const int q = 4 * kg + wave;
     if (j >= a.R || q >= m) return;
-    const float s = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
+    const float s = (float)(((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane]);
     out[(size_t)(p0 + q) * a.R + j] = BACK ? a.scale[g] * s : s;
 }
 

@@ -216,3 +216,45 @@ def test_rank_projections_at_the_edges_of_their_tiles(ctx, T, rank):
         for got, want in zip(grads[key], ref_grads[key]):
             if np.any(want):
                 assert rel_err(got, want) <= GRAD_TOL, key
+
+
+@pytest.mark.parametrize("d", [256, 1000, 1024, 2048, 4096])
+def test_rank_projections_round_as_short_sums_do(ctx, d):
+    """One token through one expert makes every adapter gradient a rank-one
+    matrix: Up's of the gate layer is (its gradient) (A x)^T, Down's of the
+    down layer (B^T g) (hidden row)^T.  Their leading singular vectors average
+    the products' own rounding away and leave that of the projections A x and
+    B^T g over d values.  Sums of 16 products added in 64 bits, rounded once to
+    32, stay below 1e-7 (half an ulp of the results alone is 3e-8 on average;
+    a model of 16 sequential roundings gives 8e-8); one serial fp32 sum per
+    quarter grows with d, 2.9e-7 at 1024 and 5.7e-7 at 4096 values."""
+    say(f"rounding of the rank projections, d={d}")
+    rank = 64
+    spec = make_moe(gt.encode_rows, d=d, h=64, E=1, k=1, S=0, precision=INT8, seed=61, std=0.05, bias_std=0.02)
+    rng = np.random.default_rng(62)
+    f32 = lambda v: v.astype(np.float32).astype(np.float64)
+    adapters = lora.make_adapters(spec, rank, 2.0 * rank, rng, up_scale=0.05)
+    for ad in adapters.values():
+        ad.down, ad.up = f32(ad.down), f32(ad.up)
+    m = with_adapters(ctx, spec, adapters, rank, 2.0 * rank)
+    got, want = {"u": [], "t": []}, {"u": [], "t": []}
+    try:
+        for _ in range(16):
+            x, G = f32(rng.standard_normal((1, d))), f32(rng.standard_normal((1, d)))
+            m.zero_adapter_gradients()
+            m.forward(x)
+            m.backward(G)
+            up = m.adapter_gradients("routed", 0, "gate")[1]
+            down = m.adapter_gradients("routed", 0, "down")[0]
+            for key, mat, exact in (("u", up, adapters[("routed", 0, "gate")].down @ x[0]),
+                                    ("t", down.T, adapters[("routed", 0, "down")].up.T @ G[0])):
+                v = np.linalg.svd(mat, full_matrices=False)[2][0]
+                got[key].append(v * (v @ exact))
+                want[key].append(exact)
+    finally:
+        m.destroy()
+    for key in got:
+        g, w = np.array(got[key]), np.array(want[key])
+        e = np.linalg.norm(g - w) / np.linalg.norm(w)
+        say(f"[d={d}] {key}: relative error {e:.2e}")
+        assert e <= 1e-7, (key, e)
