@@ -384,8 +384,11 @@ __global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const flo
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
+                        // past the last value both are zero: a zero times an
+                        // infinite row of B would be NaN
                         const float v = row[min(n + e, nval - 1)];
                         x[q][e] = n + e < nval ? v : 0.f;
+                        w[q][e] = n + e < nval ? w[q][e] : 0.f;
                     }
                 }
             } else {  // padded rows of kin values, a multiple of 64

@@ -258,3 +258,32 @@ def test_rank_projections_round_as_short_sums_do(ctx, d):
         e = np.linalg.norm(g - w) / np.linalg.norm(w)
         say(f"[d={d}] {key}: relative error {e:.2e}")
         assert e <= 1e-7, (key, e)
+
+
+@pytest.mark.parametrize("d,row", [(37, 36), (48, 47), (48, 11)])
+def test_an_infinite_row_of_up(ctx, d, row):
+    """An infinite value in one row of the down layer's Up makes that rank of
+    t = s g Up infinite with the sign of the row's gradient, and with it a row
+    of Down's gradients; 37 rows end inside a step of 16 values, whose rest adds
+    nothing."""
+    say(f"infinite Up value, d={d} row={row}")
+    spec = make_moe(gt.encode_rows, d=d, h=32, E=1, k=1, S=0, precision=INT8, seed=63, std=0.1, bias_std=0.02)
+    rng = np.random.default_rng(64)
+    adapters = lora.make_adapters(spec, 4, 8.0, rng, up_scale=0.05)
+    adapters[("routed", 0, "down")].up[row, 2] = np.inf
+    x, G = rng.uniform(-1, 1, (1, d)), rng.uniform(-1, 1, (1, d))
+    m = with_adapters(ctx, spec, adapters, 4, 8.0)
+    try:
+        m.forward(x)
+        m.backward(G)
+        got = m.adapter_gradients("routed", 0, "down")[0]
+    finally:
+        m.destroy()
+    _, st = lora.forward(spec, adapters, x)
+    want = lora.zero_grads(spec, adapters)
+    with np.errstate(all="ignore"):
+        lora.backward(spec, adapters, st, G, want)
+    want = want[("routed", 0, "down")][0]
+    assert np.all(np.isinf(want[2])) and np.all(np.isfinite(want[[0, 1, 3]]))
+    assert np.array_equal(got[2], want[2])
+    assert rel_err(got[[0, 1, 3]], want[[0, 1, 3]]) <= GRAD_TOL
