@@ -757,21 +757,36 @@ __global__ __launch_bounds__(256) void gather_input_grad_kernel(const float *__r
     dx[(size_t)t * d + i] = acc;
 }
 
-// dx[t][i] += sum_e lg[t][e] * W[e][i] (the router's base rows, fp32, row
-// stride ldw), i < d
-__global__ __launch_bounds__(256) void router_input_grad_kernel(const float *__restrict__ lg, int E,
+// dx[t][i] = sum_e lg[t][e] * W[e][i] (the router's base rows, fp32, row
+// stride ldw), i < d, over every expert: an unchosen expert's zero times an
+// infinite or NaN weight is NaN, as in any sum over all outputs.  A thread
+// takes its column for four tokens, so that the router's rows are read once
+// for them.
+constexpr int kRouterGradTokens = 4;
+
+__global__ __launch_bounds__(256) void router_input_grad_kernel(const float *__restrict__ lg, int T, int E,
                                                                 const float *__restrict__ w, int ldw, int d,
                                                                 float *__restrict__ dx, int ld_dx)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    const int t = blockIdx.y;
+    const int t0 = blockIdx.y * kRouterGradTokens;
     if (i >= d) return;
-    float s = 0.f;
-    for (int e = 0; e < E; ++e) {
-        const float l = lg[(size_t)t * E + e];
-        if (l != 0.f) s = fmaf(l, w[(size_t)e * ldw + i], s);  // uniform: zero but for the chosen experts
+    const float *l[kRouterGradTokens];
+    float s[kRouterGradTokens];
+#pragma unroll
+    for (int u = 0; u < kRouterGradTokens; ++u) {
+        l[u] = lg + (size_t)min(t0 + u, T - 1) * E;
+        s[u] = 0.f;
     }
-    dx[(size_t)t * ld_dx + i] = s;
+#pragma unroll 8
+    for (int e = 0; e < E; ++e) {
+        const float v = w[(size_t)e * ldw + i];
+#pragma unroll
+        for (int u = 0; u < kRouterGradTokens; ++u) s[u] = fmaf(l[u][e], v, s[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kRouterGradTokens; ++u)
+        if (t0 + u < T) dx[(size_t)(t0 + u) * ld_dx + i] = s[u];
 }
 
 __global__ __launch_bounds__(256) void add_rows_f64_kernel(const float *__restrict__ src, int ld, int d, int T,
@@ -942,7 +957,8 @@ hipError_t launch_router_input_grad(const float *lg, int T, int E, const float *
                                     int ld_dx, hipStream_t s)
 {
     if (T <= 0) return hipSuccess;
-    hipLaunchKernelGGL(router_input_grad_kernel, cols_grid(d, T), dim3(256), 0, s, lg, E, w, ldw, d, dx, ld_dx);
+    hipLaunchKernelGGL(router_input_grad_kernel, cols_grid(d, (T + kRouterGradTokens - 1) / kRouterGradTokens),
+                       dim3(256), 0, s, lg, T, E, w, ldw, d, dx, ld_dx);
     return hipGetLastError();
 }
 

@@ -287,3 +287,35 @@ def test_an_infinite_row_of_up(ctx, d, row):
     assert np.all(np.isinf(want[2])) and np.all(np.isfinite(want[[0, 1, 3]]))
     assert np.array_equal(got[2], want[2])
     assert rel_err(got[[0, 1, 3]], want[[0, 1, 3]]) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("T", [1, 6])
+def test_an_infinite_weight_of_an_unchosen_router_row(ctx, T):
+    """Router row 3 holds -inf in a column whose inputs are positive, so no
+    token chooses expert 3 and the forward is finite.  That column's input
+    gradient is a sum over every expert, NaN from the zero logit gradient times
+    the weight; the other columns' are not touched by it."""
+    say(f"infinite router weight, T={T}")
+    d, column = 40, 7
+    spec = make_moe(gt.encode_rows, d=d, h=24, E=4, k=2, S=1, precision=INT8, seed=71, std=0.1, router_std=0.1,
+                    bias_std=0.02)
+    spec.router.weights.values[3, column] = -np.inf
+    rng = np.random.default_rng(72)
+    adapters = lora.make_adapters(spec, 4, 8.0, rng, up_scale=0.05)
+    x, G = rng.uniform(-1, 1, (T, d)), rng.uniform(-1, 1, (T, d))
+    x[:, column] = rng.uniform(0.1, 1, T)
+    m = with_adapters(ctx, spec, adapters, 4, 8.0)
+    try:
+        y = m.forward(x)
+        r = m.last_routing()
+        dx = m.backward(G)
+    finally:
+        m.destroy()
+    assert not np.any(r.chosen == 3)
+    with np.errstate(all="ignore"):
+        ref_y, st = lora.forward(spec, adapters, x, chosen=r.chosen)
+        ref_dx = lora.backward(spec, adapters, st, G, lora.zero_grads(spec, adapters))
+    others = np.arange(d) != column
+    assert rel_err(y, ref_y) <= FWD_TOL
+    assert np.all(np.isnan(dx[:, column]))
+    assert rel_err(dx[:, others], ref_dx[:, others]) <= GRAD_TOL
