@@ -557,7 +557,7 @@ struct PendingCombine {
 // would also have to do the previous stack layer's combine.
 bool routes_fused(const gtmoe_layer *L, int T, bool f64, bool pending)
 {
-    return fused_route_fits(T, L->k, L->dp, !f64 && !pending && !L->desc.use_hash_routing && L->d % 4 == 0);
+    return fused_route_fits(T, L->k, L->E, L->dp, !f64 && !pending && !L->desc.use_hash_routing && L->d % 4 == 0);
 }
 
 // Input preparation, routing and dispatch.  Few tokens: one fused launch.

@@ -112,7 +112,7 @@ hipError_t launch_topk(const double *logits, int T, int E, int k, const double *
                        double *gates, float *gates32, hipStream_t s, int32_t *chunk_cnt = nullptr);
 hipError_t launch_hash_route(const int64_t *ids, int T, int E, int k, int32_t *chosen, double *gates,
                              float *gates32, hipStream_t s);
-bool fused_route_fits(int T, int k, int kp, bool pair);
+bool fused_route_fits(int T, int k, int E, int kp, bool pair);
 hipError_t launch_route_fused(const FusedArgs &a, bool input_f64, bool hash, bool dispatch, hipStream_t s);
 // Dispatch: one workgroup up to 1024 tokens, else (dispatch_chunked) a
 // count and a placement launch over chunks of tokens using chunk_cnt

@@ -1239,7 +1239,8 @@ hipError_t launch_dispatch(const int32_t *chosen, int T, int k, int E, int S, in
 // ---------------------------------------------------------------------------
 constexpr int kFusedMaxTK = 2048;  // T*k handled by the two-launch routing
 constexpr int kPairTokens = 256;   // more tokens: two per workgroup, where route_pair_kernel takes them
-constexpr int kPairMaxTK = 4096;   // T*k it is launched for
+constexpr int kPairMaxTK = 4096;   // T*k it is launched for with at most kPairMaxExperts experts
+constexpr int kPairMaxExperts = 64;
 constexpr int kPairMaxK = 2048;    // padded row width it holds
 
 __device__ __forceinline__ uint16_t bf16_bits(float f)
@@ -1802,12 +1803,18 @@ static hipError_t launch_pair(const FusedArgs &a, hipStream_t s)
 // beat the router, top-k and conversion launches up to T k = 4096 (d = 2048, h =
 // 1024, 64 + 1 FP4 experts, k = 4: 513 tokens 128.7 -> 121.8 us, 1000 170.4 ->
 // 164.5; d = 1024, k = 6, 500 tokens 70.0 -> 59.7; d = 1000, 14 + 2 experts, k
-// = 3, 777 87.5 -> 80.6; layer times, one sweep per limit).  Beyond, the layers
+// = 3, 777 87.5 -> 80.6; layer times, one sweep per limit), with at most 64
+// experts: every workgroup reads the whole router, and over 128 and 256 experts
+// the staged launches win (h = 64, k = 4, 1000 tokens: 64 experts staged 40.5,
+// 55.4 and 77.3 us at d = 512, 1024 and 2048, paired 39.1, 49.3 and 71.7; 128
+// experts 42.1, 56.1 and 80.9 against 45.8, 56.4 and 85.8; 256 experts 43.2,
+// 56.9 and 81.0 against 58.6, 72.0 and 112.1).  Beyond 4096 choices the layers
 // differ: k = 6, 1000 tokens 88.0 -> 84.0, but d = 2048, 128 experts, k = 8, 600
 // tokens 224-232 -> 237 and 1000 256-258 -> 270 (ranges: two runs of one route).
-bool fused_route_fits(int T, int k, int kp, bool pair)
+bool fused_route_fits(int T, int k, int E, int kp, bool pair)
 {
-    const int limit = pair && T > kPairTokens && kp <= kPairMaxK ? kPairMaxTK : kFusedMaxTK;
+    const bool wide = pair && T > kPairTokens && E <= kPairMaxExperts && kp <= kPairMaxK;
+    const int limit = wide ? kPairMaxTK : kFusedMaxTK;
     return T >= 1 && T * k <= limit && T <= 1024 && kp <= 4096;
 }
 
@@ -1848,7 +1855,7 @@ static hipError_t launch_token_typed(const FusedArgs &a, bool hash, hipStream_t 
 hipError_t launch_route_fused(const FusedArgs &a, bool input_f64, bool hash, bool dispatch, hipStream_t s)
 {
     const bool pair = !input_f64 && !hash && !a.pend_slot && a.d % 4 == 0;
-    if (!fused_route_fits(a.T, a.k, a.kp, pair)) return hipErrorInvalidValue;
+    if (!fused_route_fits(a.T, a.k, a.E, a.kp, pair)) return hipErrorInvalidValue;
     // more than one part needs the arrival counts, and a pending combine
     // then must not be written in place
     if (a.parts < 1 || (a.parts > 1 && (hash || !a.part_cnt || (a.pend_slot && (!a.x_out || a.x_out == a.x)))))

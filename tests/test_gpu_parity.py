@@ -665,7 +665,8 @@ def test_scores_that_share_their_upper_bits(ctx, E, k):
         assert np.array_equal(got.gates.view(np.int64), want.gates.view(np.int64))
 
 
-@pytest.mark.parametrize("d,E,k", [(64, 5, 2), (260, 128, 7), (1024, 16, 2), (1500, 200, 3), (2048, 64, 4)])
+@pytest.mark.parametrize("d,E,k", [(64, 5, 2), (260, 64, 7), (260, 128, 4), (1024, 16, 2), (1500, 200, 3),
+                                   (2048, 64, 4)])
 @pytest.mark.parametrize("T", [257, 258, 511])
 def test_two_tokens_per_routing_workgroup(ctx, d, E, k, T):
     """More than 256 tokens route two per workgroup: choices, gates and
@@ -692,6 +693,78 @@ def test_two_tokens_per_routing_workgroup(ctx, d, E, k, T):
     yp, cp, gp, sx, sc, sg = (np.concatenate(v, axis=1 if v[0].ndim == 3 else 0) for v in zip(*parts))
     assert np.array_equal(r.chosen, cp) and np.array_equal(r.gates, gp) and np.array_equal(y, yp)
     assert np.array_equal(s[1], sc) and np.array_equal(s[2], sg) and np.array_equal(s[0], sx)
+
+
+@pytest.mark.parametrize("T,k,E", [(512, 8, 20), (513, 8, 20), (1023, 4, 20), (1024, 4, 64), (1024, 5, 20),
+                                   (512, 4, 65), (513, 4, 65)])
+def test_paired_routing_around_its_limit(ctx, T, k, E):
+    """Two tokens per routing workgroup up to 4096 choices (2048 with more than
+    64 experts), with every
+    token-wave of the one-workgroup dispatch behind it, and the staged launches
+    just past the limit.  Up to it choices, gates and outputs are to the bit
+    those of calls of at most 256 tokens; the staged router adds its products
+    in another order, so past it near-ties may fall the other way and the gates
+    agree to fp32 logits' rounding."""
+    d = 96
+    say(f"paired routing limit T={T} k={k} E={E}")
+    spec = make_moe(gt.encode_rows, d=d, h=16, E=E, k=k, S=1, precision=INT8, seed=63, std=0.1, router_std=0.2)
+    x = np.random.default_rng(64).normal(size=(T, d))
+    m = gt.MixtureOfExperts.from_spec(ctx, spec)
+    try:
+        y = m.forward(x, path=gt.PATH_BF16)
+        r = m.last_routing()
+        parts = []
+        for rows in np.array_split(x, -(-T // 256)):
+            yp = m.forward(rows, path=gt.PATH_BF16)
+            rp = m.last_routing()
+            parts.append((yp, rp.chosen, rp.gates))
+    finally:
+        m.destroy()
+    yp, cp, gp = (np.concatenate(v) for v in zip(*parts))
+    table = oracle.dispatch(r.chosen, E)
+    assert np.array_equal(r.load, table.load)
+    assert np.array_equal(r.offsets, table.offsets)
+    assert np.array_equal(r.rows, table.rows)
+    if T * k <= (4096 if E <= 64 else 2048):
+        assert np.array_equal(r.chosen, cp) and np.array_equal(r.gates, gp) and np.array_equal(y, yp)
+    else:
+        check_routing(r.chosen, spec, x, k, f"staged T={T} k={k}")
+        same = np.all(r.chosen == cp, axis=1)
+        assert rel_err(r.gates[same], gp[same]) <= 1e-5
+        ref = oracle.moe_forward_routed(spec, x, r.chosen, r.gates)
+        assert rel_err(y, ref.outputs) <= 2e-2  # the bf16 path's bar
+
+
+@pytest.mark.parametrize("E,k", [(20, 3), (128, 6), (200, 2)])
+def test_paired_routing_with_nan_scores(ctx, E, k):
+    """Two NaN balance biases make every token of a pair take the sort, whose
+    scratch shares the two logit rows; rows with a NaN input stand first, second
+    and both in their pairs.  To the bit as in calls of one token per
+    workgroup."""
+    T, d = 300, 96
+    say(f"paired routing with NaN scores E={E} k={k}")
+    balance = np.random.default_rng(65).normal(0, 0.05, E)
+    balance[[2, E // 2]] = np.nan
+    spec = make_moe(gt.encode_rows, d=d, h=16, E=E, k=k, S=1, precision=INT8, seed=66, std=0.1, router_std=0.2,
+                    balance=balance)
+    x = np.random.default_rng(67).normal(size=(T, d))
+    x[[4, 11, 20, 21, 299], [0, 95, 50, 3, 17]] = np.nan
+    m = gt.MixtureOfExperts.from_spec(ctx, spec)
+    try:
+        y = m.forward(x, path=gt.PATH_BF16)
+        r = m.last_routing()
+        parts = []
+        for rows in np.array_split(x, 2):
+            yp = m.forward(rows, path=gt.PATH_BF16)
+            rp = m.last_routing()
+            parts.append((yp, rp.chosen, rp.gates))
+    finally:
+        m.destroy()
+    yp, cp, gp = (np.concatenate(v) for v in zip(*parts))
+    assert np.array_equal(r.chosen, cp)
+    assert same_gates(r.gates, gp)
+    assert np.array_equal(y, yp, equal_nan=True)
+    assert np.all(np.isfinite(np.delete(y, [4, 11, 20, 21, 299], axis=0)))
 
 
 @pytest.mark.parametrize("prec", [FLOAT32, INT8, FP4])
