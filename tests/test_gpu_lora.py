@@ -56,8 +56,8 @@ CASES = {
     "C2 int8 decode": (1024, 2048, 16, 2, 0, INT8, 0.0, False, 8),
     "C3 fp4 layer": (1024, 512, 64, 6, 1, FP4, 0.0, False, 64),
     # many positions per group: the transposed product on the matrix cores
-    # (32-position tiles, the down layer's rows in sixteen chunks) and dx's
-    # eight positions per thread
+    # (32-position tiles, the down layer's rows in sixteen chunks) and full
+    # tiles of 64 positions in the adapters' kernels
     "many positions per expert": (1024, 128, 4, 1, 1, INT8, 0.0, False, 1024),
     # the matrix-core product over FP4 rows with a partial last panel (d = 200
     # rows of the down layer, its gradient rows 200 floats apart) and half a
@@ -67,8 +67,8 @@ CASES = {
     # fourteen positions per group on average: eight-position tiles
     "eight-position tiles": (96, 64, 8, 2, 0, INT8, 0.0, False, 56),
 }
-# adapter rank per case (4 unless listed): sixteen ranks take the float4 runs
-# of t = s g Up, five the scalar paths
+# adapter rank per case (4 unless listed): 16 fill a block of the projections'
+# ranks, five are read one at a time
 RANKS = {"many positions per expert": 16, "small fp4 two shared": 5, "clamped": 16}
 
 
@@ -186,10 +186,12 @@ def test_adapter_errors_mirror_the_reference(ctx):
 @pytest.mark.parametrize("rank", [3, 16, 17, 20])
 @pytest.mark.parametrize("T", [1, 15, 17, 63, 65, 130])
 def test_rank_projections_at_the_edges_of_their_tiles(ctx, T, rank):
-    """Hash routing with one expert (T positions in its group and T in the
-    shared expert's) and the router's T tokens: blocks of 16 positions and tiles
-    of 64, partly filled; ranks below, at and past 16; output-gradient rows 37
-    floats apart, hidden widths that are not multiples of 16."""
+    """One routed expert (T positions in its group and T in the shared
+    expert's): blocks of 16 positions and tiles of 64, partly filled; ranks
+    below, at and past 16; output-gradient rows 37 floats apart, hidden widths
+    that are not multiples of 16.  The only expert's gate is 1 whatever its
+    logit, so the router's gradients are exactly zero; its adapter is tested
+    below."""
     d, h = 37, 53
     say(f"rank projections T={T} rank={rank}")
     spec = make_moe(gt.encode_rows, d=d, h=h, E=1, k=1, S=1, precision=INT8, seed=51, std=0.1, router_std=0.1,
@@ -216,6 +218,46 @@ def test_rank_projections_at_the_edges_of_their_tiles(ctx, T, rank):
         for got, want in zip(grads[key], ref_grads[key]):
             if np.any(want):
                 assert rel_err(got, want) <= GRAD_TOL, key
+            else:
+                assert not np.any(got), key
+
+
+@pytest.mark.parametrize("rank", [3, 16, 17, 20])
+@pytest.mark.parametrize("T", [1, 15, 17, 63, 65, 130])
+def test_router_adapter_at_the_edges_of_its_tiles(ctx, T, rank):
+    """The router's adapter over its own tiles of the T tokens: 21 experts, so
+    that its rank is not cut below 20, three of them chosen.  Its projection
+    decides the gates (forward outputs) and takes a gradient from them, and its
+    input gradients join the layer's."""
+    d, h, E, k = 37, 53, 21, 3
+    say(f"router adapter T={T} rank={rank}")
+    spec = make_moe(gt.encode_rows, d=d, h=h, E=E, k=k, S=1, precision=INT8, seed=53, std=0.1, router_std=0.1,
+                    bias_std=0.02)
+    rng = np.random.default_rng(54 + T)
+    alpha = 2.0 * rank
+    adapters = lora.make_adapters(spec, rank, alpha, rng, up_scale=0.3)
+    x = rng.uniform(-1, 1, (T, d))
+    G = rng.uniform(-1, 1, (T, d))
+    m = with_adapters(ctx, spec, adapters, rank, alpha)
+    try:
+        y = m.forward(x)
+        r = m.last_routing()
+        dx = m.backward(G)
+        down, up = m.adapter_gradients("router", 0)
+    finally:
+        m.destroy()
+    ref_y, st = lora.forward(spec, adapters, x, None, chosen=r.chosen)
+    ref_grads = lora.zero_grads(spec, adapters)
+    ref_dx = lora.backward(spec, adapters, st, G, ref_grads)
+    want_down, want_up = ref_grads[("router", 0, None)]
+    assert down.shape == (rank, d) and np.any(want_down) and np.any(want_up)
+    assert rel_err(r.gates, st.gates) <= FWD_TOL
+    assert rel_err(y, ref_y) <= FWD_TOL
+    assert rel_err(dx, ref_dx) <= GRAD_TOL
+    assert rel_err(down, want_down) <= GRAD_TOL
+    assert rel_err(up, want_up) <= GRAD_TOL
+    idle = ~np.isin(np.arange(E), r.chosen)  # no token chose them: their rows of Up's gradients
+    assert not np.any(up[idle])
 
 
 @pytest.mark.parametrize("d", [256, 1000, 1024, 2048, 4096])

@@ -323,8 +323,8 @@ def test_device_forward_folds_two_term_combine(ctx, name, cfg, prec, T):
 @pytest.mark.parametrize("d,h,T", [(4096, 192, 16), (192, 4096, 64)])
 def test_widest_decode_gemv(ctx, d, h, T):
     """The fp32 path at its widest K (4096): the gate/up (d) or down (h)
-    kernel stages 8 tokens x 4096 values as bf16 hi/lo (128 KiB of LDS) plus
-    the self-dispatch entry list."""
+    kernel's waves stream 16 chunks of 64 values each, its LDS holding the
+    partial sums and the self-dispatch entry list."""
     say(f"widest GEMV d={d} h={h} T={T}")
     spec = make_moe(gt.encode_rows, d=d, h=h, E=6, k=3, S=1, precision=FP4, seed=15, std=0.02, bias_std=0.01)
     x = np.random.default_rng(16).uniform(-1, 1, (T, d))
@@ -338,8 +338,8 @@ def test_widest_decode_gemv(ctx, d, h, T):
 
 @pytest.mark.parametrize("E,k", [(16, 3), (64, 4), (96, 2)])
 def test_decode_routing_ties_and_nan_match_the_oracle(ctx, E, k):
-    """The decode routing kernel (ranked choice for E <= 64, rounds of
-    arg-max above) on logits with exact ties and NaN: a router of zero
+    """The decode routing kernel (k rounds on the scores' keys, a sort where a
+    score is NaN) on logits with exact ties and NaN: a router of zero
     weights makes every logit of a token equal to its bias, and a NaN input
     makes a token's logits NaN.  Chosen experts and gates are bit-exact
     against the oracle's routing of the same float64 logits."""
