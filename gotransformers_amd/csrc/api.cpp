@@ -263,7 +263,6 @@ struct TrainWorkspace {
     char *tables = nullptr;
     int32_t *pgroup = nullptr;  // [P]
     int4 *tiles_tr = nullptr;  // [P + G]
-    int32_t *goff_router = nullptr;  // {0, T}
     double *zero_bias = nullptr;     // [E]
     float *partial = nullptr;        // [chunks][P][max(dp, hp)] row-chunk sums of the transposed product
     int chunks = 1;                  // row chunks the partial buffer holds
@@ -1164,7 +1163,7 @@ size_t train_tables_bytes(const gtmoe_layer *L, int cap)
 {
     const size_t P = (size_t)cap * (L->S + L->k), G = L->G, n = lora_outer_tile_positions();
     return 4 * P + 16 * (P + G) + (16 * (P / n + G) + 4 * (G + 1) + 4 * G) + (16 * ((size_t)cap / n + 1) + 4 * 2 + 4) +
-           4 * 2 + 9 * 64;
+           8 * 64;
 }
 
 int32_t ensure_train_workspace(gtmoe_layer *L, int T)
@@ -1214,8 +1213,7 @@ int32_t ensure_train_workspace(gtmoe_layer *L, int T)
     return GTMOE_OK;
 }
 
-LoraArgs lora_args(const AdapterSet &a, int P, const int32_t *pgroup, const int32_t *goff,
-                   const TrainWorkspace::OuterTiles *ot = nullptr)
+LoraArgs lora_args(const AdapterSet &a, int P, const TrainWorkspace::OuterTiles &ot)
 {
     LoraArgs l{};
     l.A = a.A;
@@ -1225,17 +1223,12 @@ LoraArgs lora_args(const AdapterSet &a, int P, const int32_t *pgroup, const int3
     l.kin = a.kin;
     l.width = a.width;
     l.rows = a.rows;
-    l.G = a.G;
     l.P = P;
-    l.pgroup = pgroup;
-    l.goff = goff;
-    if (ot) {
-        l.otiles = ot->tiles;
-        l.otoff = ot->toff;
-        l.notiles = ot->n;
-        l.omulti = ot->multi;
-        l.nomulti = ot->nmulti;
-    }
+    l.otiles = ot.tiles;
+    l.otoff = ot.toff;
+    l.notiles = ot.n;
+    l.omulti = ot.multi;
+    l.nomulti = ot.nmulti;
     return l;
 }
 
@@ -1345,11 +1338,10 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
     if (hash) {
         RUN(ctx, s, "hash_route", launch_hash_route(w.ids, T, E, k, w.chosen, w.gates, w.gates32, s));
     } else {
-        tw.goff_router = tables.put(std::vector<int32_t>{0, T});
         put_outer_tiles(tables, {0, T}, tw.rt);
         HIP_TRY(ctx, tables.send(s));
         RUN(ctx, s, "router", launch_router(w.xf, dp, T, d, L->router_w, dp, tw.zero_bias, E, w.logits, s));
-        const LoraArgs ar = lora_args(L->ad_router, T, nullptr, tw.goff_router, &tw.rt);
+        const LoraArgs ar = lora_args(L->ad_router, T, tw.rt);
         RUN(ctx, s, "lora_down", launch_lora_down(ar, w.xf, dp, nullptr, tw.u_router, s));
         RUN(ctx, s, "lora_up_bias", launch_lora_up_bias_f64(ar, tw.u_router, w.logits, E, L->router_b, s));
         RUN(ctx, s, "topk", launch_topk(w.logits, T, E, k, L->balance, w.chosen, w.gates, w.gates32, s));
@@ -1420,7 +1412,7 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
         float *pre, *u;
     };
     for (const Role &r : {Role{L->gate, L->ad_gate, tw.gpre, tw.u_gate}, Role{L->up, L->ad_up, tw.upre, tw.u_up}}) {
-        const LoraArgs la = lora_args(r.a, P, tw.pgroup, w.goff, &tw.ot);
+        const LoraArgs la = lora_args(r.a, P, tw.ot);
         RUN(ctx, s, "lora_down", launch_lora_down(la, w.xf, dp, w.tok, r.u, s));
         RUN(ctx, s, "lora_up_bias", launch_lora_up_bias(la, r.u, r.pre, hp, r.m.biases, s));
     }
@@ -1443,7 +1435,7 @@ int32_t adapter_forward(gtmoe_layer *L, int T, const double *inputs, const int64
     b.ld_out = d;
     b.raw = 1;
     RUN(ctx, s, "gemv_down", launch_gemv_down(b, L->down.precision, slices, s));
-    const LoraArgs ld = lora_args(L->ad_down, P, tw.pgroup, w.goff, &tw.ot);
+    const LoraArgs ld = lora_args(L->ad_down, P, tw.ot);
     RUN(ctx, s, "lora_down", launch_lora_down(ld, w.hidden32, hp, nullptr, tw.u_down, s));
     RUN(ctx, s, "lora_up_bias", launch_lora_up_bias(ld, tw.u_down, w.slot_out, d, L->down.biases, s));
     RUN(ctx, s, "combine",
@@ -1486,7 +1478,7 @@ int32_t adapter_backward(gtmoe_layer *L, int T, const double *output_grads, doub
     };
     RUN(ctx, s, "rows_transposed", transposed(L->down, tw.eg, d, tw.hgrad, hp));
     RUN(ctx, s, "lora_backward",
-        launch_lora_backward(lora_args(L->ad_down, P, tw.pgroup, w.goff, &tw.ot), tw.eg, d,
+        launch_lora_backward(lora_args(L->ad_down, P, tw.ot), tw.eg, d,
                              tw.u_down, w.hidden32, hp, nullptr, tw.t, tw.hgrad, hp, L->ad_down.dA, L->ad_down.dB,
                              tw.outer, s));
     RUN(ctx, s, "swiglu_backward",
@@ -1500,7 +1492,7 @@ int32_t adapter_backward(gtmoe_layer *L, int T, const double *output_grads, doub
                           Role{L->up, L->ad_up, tw.ugrad, tw.u_up, tw.dxu}}) {
         RUN(ctx, s, "rows_transposed", transposed(r.m, r.grad, hp, r.dx, dp));
         RUN(ctx, s, "lora_backward",
-            launch_lora_backward(lora_args(r.a, P, tw.pgroup, w.goff, &tw.ot), r.grad, hp,
+            launch_lora_backward(lora_args(r.a, P, tw.ot), r.grad, hp,
                                  r.u, w.xf, dp, w.tok, tw.t, r.dx, dp, r.a.dA, r.a.dB, tw.outer, s));
     }
     RUN(ctx, s, "gather_input_grad", launch_gather_input_grad(tw.dxg, tw.dxu, dp, d, T, S, k, w.pos, tw.dx, s));
@@ -1510,7 +1502,7 @@ int32_t adapter_backward(gtmoe_layer *L, int T, const double *output_grads, doub
                                    tw.lgf, s));
         RUN(ctx, s, "router_input_grad", launch_router_input_grad(tw.lgf, T, E, L->router_w, dp, d, tw.dxr, dp, s));
         RUN(ctx, s, "lora_backward",
-            launch_lora_backward(lora_args(L->ad_router, T, nullptr, tw.goff_router, &tw.rt),
+            launch_lora_backward(lora_args(L->ad_router, T, tw.rt),
                                  tw.lgf, E, tw.u_router, w.xf, dp, nullptr, tw.t, tw.dxr, dp, L->ad_router.dA,
                                  L->ad_router.dB, tw.outer, s));
         RUN(ctx, s, "add_rows", launch_add_rows_f64(tw.dxr, dp, d, T, tw.dx, s));

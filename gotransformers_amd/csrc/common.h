@@ -105,12 +105,13 @@ struct GemvArgs {
     const float *gates32;    // [T][k]
     int T, k, S;
     // Few tokens (self_dispatch): no dispatch tables.  Grid row y < S *
-    // shared_slices is a slice of 8 tokens of a shared expert; the next 2E
-    // rows are two workgroups per routed expert e (rows y and y + E), which
-    // find e's (token, slot) entries in `chosen` and take every other pass
-    // of 8.  Rows are indexed directly: shared expert s, token t at s*T + t;
+    // shared_slices is a slice of 8 tokens of a shared expert; the next E rows
+    // are the routed experts, each of which finds its (token, slot) entries in
+    // `chosen` and takes the first 8; the T k / 8 rows after them take whatever
+    // the experts hold beyond, 8 entries a row.  Rows are indexed directly: shared expert s, token t at s*T + t;
     // routed entry t*k + j at S*T + t*k + j.  list_off: LDS offset of the
-    // entry list (set by the launcher; room for T*k entries).
+    // entry list (set by the launcher; room for T*k entries, two ints and a
+    // count per expert).
     int self_dispatch, shared_slices, list_off, E;
     // raw: write the bare products, no bias or activation (gate to out, up to
     // raw_up with the same layout); the adapter path's forward

@@ -171,13 +171,13 @@ __device__ __forceinline__ f32x4 mfma4(s16x4 a, s16x4 b, f32x4 c)
 __device__ __forceinline__ float silu(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 
 // Codes (and scales) of chunk ch of the lane's row, for every matrix.  A
-// chunk of CB blocks starts at block ch*CB; its scales are CB consecutive
-// floats of the row's 4-block scale group.  vo = lane * 16; ch is uniform
-// across the wave.
+// chunk of scaled codes is one 4-block scale group.  vo = lane * 16; ch is
+// uniform across the wave.
 template <int PREC, int MATS>
 __device__ __forceinline__ void load_chunk(ChunkRegs<PREC, MATS> &r, const PanelSrc (&src)[MATS], uint32_t vo, int ch)
 {
-    constexpr int U = Chunk<PREC>::U, CB = Chunk<PREC>::CB;
+    constexpr int U = Chunk<PREC>::U;
+    static_assert(PREC == kFloat32 || Chunk<PREC>::CB == 4, "a chunk's scales are one 16-byte load");
 #pragma unroll
     for (int m = 0; m < MATS; ++m) {
 #pragma unroll
@@ -185,21 +185,11 @@ __device__ __forceinline__ void load_chunk(ChunkRegs<PREC, MATS> &r, const Panel
             r.c[m][u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(src[m].codes, vo,
                                                                                         (ch * U + u) * 1024, 0));
         if constexpr (PREC != kFloat32) {
-            const int b = ch * CB;
-            const int so = (b >> 2) * 1024 + (b & 3) * 4;
-            if constexpr (CB == 4) {
-                const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(src[m].scales, vo, so, 0));
-                r.s[m][0] = v.x;
-                r.s[m][1] = v.y;
-                r.s[m][2] = v.z;
-                r.s[m][3] = v.w;
-            } else if constexpr (CB == 2) {
-                const float2 v = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(src[m].scales, vo, so, 0));
-                r.s[m][0] = v.x;
-                r.s[m][1] = v.y;
-            } else {
-                r.s[m][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src[m].scales, vo, so, 0));
-            }
+            const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(src[m].scales, vo, ch * 1024, 0));
+            r.s[m][0] = v.x;
+            r.s[m][1] = v.y;
+            r.s[m][2] = v.z;
+            r.s[m][3] = v.w;
         }
     }
 }
@@ -859,13 +849,7 @@ hipError_t launch_panels(const GemvArgs &a0, int max_slices, hipStream_t s)
         a.list_off = (int)((lds + 15) / 16 * 16);
         lds = (size_t)a.list_off + ((size_t)a.T * a.k + 2 + a.E) * sizeof(int);
     }
-    if (lds > 160 * 1024) return hipErrorInvalidValue;
-    const void *fn = a.self_dispatch ? reinterpret_cast<const void *>(&gemv_kernel<PREC, GATEUP, true, MATS, NW, RING>)
-                                     : reinterpret_cast<const void *>(&gemv_kernel<PREC, GATEUP, false, MATS, NW, RING>);
-    if (lds > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
+    if (lds > 64 * 1024) return hipErrorInvalidValue;  // 32 KiB and lists of at most 512 choices and 256 experts
     constexpr int kRows = kPanelRows * (GATEUP ? 1 : MATS);  // rows of a workgroup
     const dim3 grid((a.rows + kRows - 1) / kRows, max_slices);
     if (a.self_dispatch)
@@ -923,9 +907,8 @@ hipError_t launch_few(const GemvArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-// A few tokens through a layer wide enough that gemv_kernel runs eight waves
-// over a panel (at least 16 chunks of K): the few-token kernel, with R = 16
-// rows per workgroup when that still gives 256 workgroups, else 8.  Int8 and
+// A few tokens through a layer of K >= 512 values: the few-token kernel, with
+// R = 16 rows per workgroup when that still gives 256 workgroups, else 8.  Int8 and
 // FP4 rows whose 16-byte units divide evenly among a workgroup's unit
 // phases.  Returns false (nothing launched) otherwise.
 template <bool GATEUP>

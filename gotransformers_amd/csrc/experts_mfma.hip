@@ -1,7 +1,8 @@
 // bf16 MFMA grouped GEMM for many tokens per expert (prefill).
 //
 // One workgroup computes a 128-position (few tokens per expert: 64-position,
-// mfma_tile_m) x 256-column tile of one group (expert) with v_mfma_f32_32x32x16_bf16, fp32 accumulation:
+// mfma_tile_m) x 256-column (down over few tiles: 128-column) tile of one group
+// (expert) with v_mfma_f32_32x32x16_bf16, fp32 accumulation:
 //   gate/up  A = activations gathered by token (bf16), B = 128 gate rows and
 //            the same 128 up rows of the expert, dequantized (Int8 code or
 //            e2m1 code times its fp32 block scale, rounded to bf16); the

@@ -25,12 +25,10 @@ struct RowsArgs {
 };
 
 // Low-rank adapters of one weight role over G groups (A [G][R][kin], B
-// [G][rows][R], scale [G]) applied to P positions (pgroup[p]: group of p, or
-// null: group 0; goff[G+1]: first position of every group).
+// [G][rows][R], scale [G]) applied to P positions, by tiles of one group each.
 struct LoraArgs {
     const float *A, *B, *scale;
-    int R, kin, width, rows, G, P;
-    const int32_t *pgroup, *goff;
+    int R, kin, width, rows, P;
     // tiles of at most lora_outer_tile_positions() positions of one group
     // (group, first position, positions, 1 if the group has more than one
     // tile else 0), every group's in position order, the first tile of

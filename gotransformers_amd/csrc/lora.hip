@@ -14,9 +14,9 @@
 //
 // Work is numbered by positions as in the expert kernels: P = T*(S+k), shared
 // expert s on positions [s*T, (s+1)*T), the routed (token, slot) pairs after
-// them in dispatch order; pgroup[p] is the group of position p, goff[G+1]
-// the first position of every group.  A position's input row is in_tok[p]
-// (gate/up: the token) or p itself (down: the hidden row) when in_tok is null.
+// them in dispatch order; the adapters' kernels take tiles of one group's
+// positions.  A position's input row is in_tok[p] (gate/up: the token) or p
+// itself (down: the hidden row) when in_tok is null.
 //
 // Adapter storage per weight role, all groups in one allocation, zero beyond
 // a layer's rank and beyond its widths (so the padding adds nothing):

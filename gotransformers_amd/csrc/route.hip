@@ -1217,7 +1217,7 @@ hipError_t launch_dispatch(const int32_t *chosen, int T, int k, int E, int S, in
                            int32_t *rows, int32_t *pos, int32_t *goff, int32_t *tok, int32_t *tile_off,
                            int4 *tile_desc, int32_t *chunk_cnt, hipStream_t s, bool counted)
 {
-    if (!dispatch_chunked(T)) {  // one workgroup: token-waves x experts over its 16 waves
+    if (!dispatch_chunked(T)) {  // one workgroup, a thread per token
         hipLaunchKernelGGL(dispatch_kernel, dim3(1), dim3(1024), 0, s, chosen, T, k, E, S, bm, load, offsets, rows,
                            pos, goff, tok, tile_off, tile_desc, PackParts{}, nullptr);
         return hipGetLastError();
