@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256) void sum_chunks_kernel(const float *__restrict
 // over 64 lanes: 7.6e-8 to 1.07e-7), in the same time.  Eight steps' loads are
 // in flight.  (One wave per (position, rank), or one workgroup per position,
 // read the adapter's values for every position: 3584 positions, 16 ranks, 512
-// to 1024 values 17.1 and 15.9 us per launch, 8.3 and 6.4 as here.)
+// to 1024 values 17.4 and 16.1 us per launch, 8.2 and 7.8 as here.)
 constexpr int kOpPositions = 64;  // positions of a tile at most
 constexpr int kRkPositions = 16;  // positions of a workgroup
 constexpr int kRkStep = 16;       // values per step
@@ -761,7 +761,8 @@ __global__ __launch_bounds__(256) void gather_input_grad_kernel(const float *__r
 // stride ldw), i < d, over every expert: an unchosen expert's zero times an
 // infinite or NaN weight is NaN, as in any sum over all outputs.  A thread
 // takes its column for four tokens, so that the router's rows are read once
-// for them.
+// for them (512 tokens, 64 experts, d = 1024: 25.5 us one token per thread, 6.6
+// as here).
 constexpr int kRouterGradTokens = 4;
 
 __global__ __launch_bounds__(256) void router_input_grad_kernel(const float *__restrict__ lg, int T, int E,
