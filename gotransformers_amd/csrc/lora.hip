@@ -344,13 +344,15 @@ __global__ __launch_bounds__(256) void sum_chunks_kernel(const float *__restrict
 // over 64 lanes: 7.6e-8 to 1.07e-7), in the same time.  Eight steps' loads are
 // in flight.  (One wave per (position, rank), or one workgroup per position,
 // read the adapter's values for every position: 3584 positions, 16 ranks, 512
-// to 1024 values 17.4 and 16.1 us per launch, 8.2 and 7.8 as here.)
+// to 1024 values 17.4 and 16.1 us per launch, 8.1 and 6.3 as here.)
 constexpr int kOpPositions = 64;  // positions of a tile at most
 constexpr int kRkPositions = 16;  // positions of a workgroup
 constexpr int kRkStep = 16;       // values per step
 constexpr int kRkDepth = 8;       // steps in flight
 
-template <bool BACK>
+// RAGGED (back only): gradient rows that are not 16-byte aligned or not whole
+// steps of values.
+template <bool BACK, bool RAGGED>
 __global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const float *__restrict__ in, int ld_in,
                                                            const int32_t *__restrict__ in_tok, float *__restrict__ out)
 {
@@ -362,8 +364,7 @@ __global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const flo
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, kg = lane >> 4;
     const int j = blockIdx.y * 16 + li, jc = min(j, a.R - 1);
-    const int nval = BACK ? a.rows : a.kin;
-    const bool vec = (ld_in & 3) == 0;  // BACK over output gradients: rows of any width
+    const int nval = BACK ? a.rows : a.kin;  // kin: padded rows, a multiple of 64
     const int p = p0 + min(li, m - 1);
     const float *row = in + (size_t)(in_tok ? in_tok[p] : p) * ld_in;
     const float *ad = BACK ? a.B + (size_t)g * a.rows * a.R + jc : a.A + ((size_t)g * a.R + jc) * a.kin;
@@ -374,30 +375,35 @@ __global__ __launch_bounds__(256) void lora_to_rank_kernel(LoraArgs a, const flo
         f32x4 x[kRkDepth], w[kRkDepth];
 #pragma unroll
         for (int q = 0; q < kRkDepth; ++q) {
-            // steps past the wave's last repeat it and are not multiplied
+            // steps past the wave's last repeat it and are not added
             const int n = kRkStep * min(sb + q, s1 - 1) + 4 * kg;
+            if constexpr (RAGGED) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[q][e] = row[min(n + e, nval - 1)];
+            } else {
+                x[q] = *reinterpret_cast<const f32x4 *>(row + n);
+            }
             if constexpr (BACK) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) w[q][e] = ad[(size_t)min(n + e, nval - 1) * a.R];
-                if (vec && nval % kRkStep == 0) {  // uniform
-                    x[q] = *reinterpret_cast<const f32x4 *>(row + n);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        // past the last value both are zero: a zero times an
-                        // infinite row of B would be NaN
-                        const float v = row[min(n + e, nval - 1)];
-                        x[q][e] = n + e < nval ? v : 0.f;
-                        w[q][e] = n + e < nval ? w[q][e] : 0.f;
-                    }
-                }
-            } else {  // padded rows of kin values, a multiple of 64
+            } else {
                 w[q] = *reinterpret_cast<const f32x4 *>(ad + n);
-                x[q] = *reinterpret_cast<const f32x4 *>(row + n);
             }
         }
 #pragma unroll
         for (int q = 0; q < kRkDepth; ++q) {
+            if constexpr (RAGGED) {
+                // past the last value both are zero: a zero times an infinite
+                // row of B would be NaN (selects between the loads made them
+                // wait for each other, 32 tokens of 2048 values 12.0 us a
+                // launch instead of 6.4)
+                const int n = kRkStep * min(sb + q, s1 - 1) + 4 * kg;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x[q][e] = n + e < nval ? x[q][e] : 0.f;
+                    w[q][e] = n + e < nval ? w[q][e] : 0.f;
+                }
+            }
             f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
 #pragma unroll
             for (int e = 0; e < 4; e += 2) {
@@ -863,6 +869,7 @@ int rows_transposed_colblocks(int nblocks, int tile)
 
 namespace {
 bool tiles_given(const LoraArgs &a) { return a.notiles > 0 && a.otiles && a.otoff; }
+dim3 to_rank_grid(const LoraArgs &a) { return dim3(a.notiles, (a.R + 15) / 16, kOpPositions / kRkPositions); }
 dim3 from_rank_grid(const LoraArgs &a, int columns)
 {
     return dim3((columns + 255) / 256, a.notiles, kOpPositions / kFromRank);
@@ -874,8 +881,7 @@ hipError_t launch_lora_down(const LoraArgs &a, const float *in, int ld_in, const
 {
     if (a.P <= 0 || a.R <= 0) return hipSuccess;
     if (!tiles_given(a)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(lora_to_rank_kernel<false>, dim3(a.notiles, (a.R + 15) / 16, kOpPositions / kRkPositions), dim3(256), 0, s, a, in, ld_in,
-                       in_tok, u);
+    hipLaunchKernelGGL((lora_to_rank_kernel<false, false>), to_rank_grid(a), dim3(256), 0, s, a, in, ld_in, in_tok, u);
     return hipGetLastError();
 }
 
@@ -909,8 +915,10 @@ hipError_t launch_lora_backward(const LoraArgs &a, const float *grad, int ld_g, 
     launch_outer(OuterArgs{a.otiles, u, a.R, grad, ld_g, nullptr, a.rows, nullptr, a.scale, dB,
                            (long long)a.rows * a.R, 1LL, (long long)a.R},
                  a, scratch, s);
-    hipLaunchKernelGGL(lora_to_rank_kernel<true>, dim3(a.notiles, (a.R + 15) / 16, kOpPositions / kRkPositions), dim3(256), 0, s, a, grad, ld_g,
-                       nullptr, t);
+    if (a.rows % kRkStep == 0 && ld_g % 4 == 0)
+        hipLaunchKernelGGL((lora_to_rank_kernel<true, false>), to_rank_grid(a), dim3(256), 0, s, a, grad, ld_g, nullptr, t);
+    else
+        hipLaunchKernelGGL((lora_to_rank_kernel<true, true>), to_rank_grid(a), dim3(256), 0, s, a, grad, ld_g, nullptr, t);
     // dA += t^T in: columns are the inputs i, the sums land at dA[g][j][i]
     launch_outer(OuterArgs{a.otiles, t, a.R, in, ld_in, in_tok, a.width, nullptr, nullptr, dA, (long long)a.R * a.kin,
                            (long long)a.kin, 1LL},
